@@ -1,7 +1,7 @@
 """Build libtagi_hip.so for gfx950 from csrc/*.hip with hipcc.
 
 Each translation unit compiles in its own hipcc process (in parallel; the GEMM kernel
-instantiations are split over 18 units), then one hipcc link produces ``triton_tagi_amd/libtagi_hip.so`` in-tree, next to the Python package
+instantiations are split over 42 units), then one hipcc link produces ``triton_tagi_amd/libtagi_hip.so`` in-tree, next to the Python package
 that loads it.
 
     python triton-tagi_amd/build.py            # build
@@ -51,10 +51,10 @@ def _run(cmd: list[str]) -> None:
         raise RuntimeError(f"command failed ({proc.returncode}): {' '.join(cmd)}\n{proc.stdout}")
 
 
-# tagi_gemm_inst.hip holds the GEMM kernels; it is compiled once per tile config (0..5)
+# tagi_gemm_inst.hip holds the GEMM kernels; it is compiled once per tile config (0..13)
 # and product (0..2), each into its own object.
 INST = "tagi_gemm_inst.hip"
-N_CFG, N_PROD = 6, 3
+N_CFG, N_PROD = 14, 3
 
 
 def compile_units() -> list[tuple[Path, Path, list[str]]]:

@@ -61,9 +61,10 @@ static int check_geom(const tagi_conv_geom* g, const char* what) {
 
 // zero_var: a deterministic input (Sa NULL), run as the shared-A product (mean ma mw,
 // variance ma^2 Sw; the Sa (mw^2 + Sw) terms it leaves out are exact zeros)
-static Plan conv_fwd_plan(const tagi_conv_geom* g, bool zero_var = false) {
-  return choose_plan(g->N * g->Ho * g->Wo, g->Cout, g->C * g->k * g->k, 1, zero_var ? PROD_SHARED_A : PROD_FWD, true,
-                     16);
+static Plan conv_fwd_plan(const tagi_conv_geom* g, bool zero_var = false, bool split = true) {
+  // (the split kernel's patch loads take up to 25 taps)
+  return choose_plan(g->N * g->Ho * g->Wo, g->Cout, g->C * g->k * g->k, 1, zero_var ? PROD_SHARED_A : PROD_FWD, split,
+                     split ? 16 : 1, nullptr, XD_A | (g->C % 4 ? XD_SCALAR : 0), g->Cout < 4 || g->k > 5);
 }
 
 // Largest row count (phase 0) and largest reduction over the stride phases of the
@@ -81,24 +82,28 @@ static void bwd_phase0(const tagi_conv_geom* g, int64_t* R, int64_t* K) {
   *K = kmax;
 }
 
-static Plan conv_bwd_plan(const tagi_conv_geom* g) {
+static Plan conv_bwd_plan(const tagi_conv_geom* g, bool split = true) {
   int64_t R, K;
   bwd_phase0(g, &R, &K);
   if (K <= 0) K = 1;
   const ConvG cg = to_g(g);
   const int nph = cg.stride * cg.stride;
   int64_t pk[64];
-  if (nph > 64) return choose_plan(R, g->C, K, nph, PROD_SHARED_B, true, 16);
+  const int xd = XD_A | (g->Cout % 4 ? XD_SCALAR : 0);
+  const bool narrow = g->C < 4 || g->k > 5;
+  if (!split || nph > 64)
+    return choose_plan(R, g->C, K, nph, PROD_SHARED_B, split, split ? 16 : 1, nullptr, xd, narrow);
   for (int ph = 0; ph < nph; ++ph) {
     const Phase p = make_phase(cg, ph);
     pk[ph] = (int64_t)p.nkh * p.nkw * g->Cout;
   }
-  return choose_plan(R, g->C, K, nph, PROD_SHARED_B, true, 16, pk);
+  return choose_plan(R, g->C, K, nph, PROD_SHARED_B, true, 16, pk, xd, narrow);
 }
 
 // rows: the weight rows (c, kh, kw), plus the ones row of the bias sums when the GEMM forms them
 static Plan conv_wgrad_plan(const tagi_conv_geom* g, bool bias) {
-  return choose_plan(g->C * g->k * g->k + (bias ? 1 : 0), g->Cout, g->N * g->Ho * g->Wo, 1, PROD_SHARED_A, true, 512);
+  return choose_plan(g->C * g->k * g->k + (bias ? 1 : 0), g->Cout, g->N * g->Ho * g->Wo, 1, PROD_SHARED_A, true, 512, nullptr, XD_B,
+                     g->Cout < 4);
 }
 
 static int64_t wt_floats(const tagi_conv_geom* g) { return ((g->C * g->k * g->k * g->Cout) + 3) / 4 * 4; }
@@ -156,21 +161,22 @@ static int conv_fwd_impl(const char* what, const float* ma, const float* Sa, con
   a.R = (int)R;
   a.C = (int)C;
   a.Kred = (int)K;
+  a.tile32 = g->C % 32 == 0;
   const bool va = g->C % 4 == 0 && al16(ma) && (zero_var || al16(Sa));
   const bool vb = g->Cout % 4 == 0 && al16(mw) && al16(Sw);
   if (zero_var) {
     if (va && vb && g->C % 16 == 0 && g->k <= 5)
-      return run_gemm<PROD_SHARED_A, LD_CFWD_A4T, LD_CFWD_B4T>(a, 1, p, ws, ws_bytes, s, what);
-    if (va && vb) return run_gemm<PROD_SHARED_A, LD_CFWD_A4, LD_CFWD_B4>(a, 1, p, ws, ws_bytes, s, what);
-    if (vb) return run_gemm<PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B4>(a, 1, p, ws, ws_bytes, s, what);
-    return run_gemm<PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B_S>(a, 1, p, ws, ws_bytes, s, what);
+      return run_gemm<PROD_SHARED_A, LD_CFWD_A4T, LD_CFWD_B4T, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+    if (va && vb) return run_gemm<PROD_SHARED_A, LD_CFWD_A4, LD_CFWD_B4, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+    if (vb) return run_gemm<PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B4, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+    return run_gemm<PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B_S, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
   }
   // 16 channels per k tile and at most 25 taps: the tile-aligned loaders
   if (va && vb && g->C % 16 == 0 && g->k <= 5)
-    return run_gemm<PROD_FWD, LD_CFWD_A4T, LD_CFWD_B4T>(a, 1, p, ws, ws_bytes, s, what);
-  if (va && vb) return run_gemm<PROD_FWD, LD_CFWD_A4, LD_CFWD_B4>(a, 1, p, ws, ws_bytes, s, what);
-  if (vb) return run_gemm<PROD_FWD, LD_CFWD_A_S, LD_CFWD_B4>(a, 1, p, ws, ws_bytes, s, what);
-  return run_gemm<PROD_FWD, LD_CFWD_A_S, LD_CFWD_B_S>(a, 1, p, ws, ws_bytes, s, what);
+    return run_gemm<PROD_FWD, LD_CFWD_A4T, LD_CFWD_B4T, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+  if (va && vb) return run_gemm<PROD_FWD, LD_CFWD_A4, LD_CFWD_B4, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+  if (vb) return run_gemm<PROD_FWD, LD_CFWD_A_S, LD_CFWD_B4, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
+  return run_gemm<PROD_FWD, LD_CFWD_A_S, LD_CFWD_B_S, 0, XD_A>(a, 1, p, ws, ws_bytes, s, what);
 }
 
 extern "C" int tagi_conv2d_fwd(const float* ma, const float* Sa, const float* mw, const float* Sw, const float* mb,
@@ -183,7 +189,7 @@ extern "C" int tagi_conv2d_fwd(const float* ma, const float* Sa, const float* mw
   const int64_t R = g->N * g->Ho * g->Wo, C = g->Cout, K = g->C * g->k * g->k;
   Plan p = conv_fwd_plan(g, Sa == nullptr);
   if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, R, C, 1)))
-    p = choose_plan(R, C, K, 1, Sa ? PROD_FWD : PROD_SHARED_A, false, 1);
+    p = conv_fwd_plan(g, Sa == nullptr, false);
   return conv_fwd_impl(what, ma, Sa, mw, Sw, mb, Sb, mz, Sz, g, p, nullptr, nullptr, ws, ws_bytes,
                        as_stream(stream));
 }
@@ -334,6 +340,7 @@ static int conv_bwd_delta_impl(const char* what, const float* dmz, const float* 
   a.C = (int)g->C;
   a.Kred = (int)K0;
   a.phased = 1;
+  a.tile32 = g->Cout % 32 == 0;
   {
     // longest phase reductions first (stable for equal lengths)
     int64_t kz[64];
@@ -352,7 +359,7 @@ static int conv_bwd_delta_impl(const char* what, const float* dmz, const float* 
   Plan p = conv_bwd_plan(g);
   float* part = ws + wt_floats(g);
   const int64_t part_bytes = ws_bytes - wt_floats(g) * (int64_t)sizeof(float);
-  if (p.splits > 1 && part_bytes < plan_ws_bytes(p, R0, g->C, nph)) p = choose_plan(R0, g->C, K0, nph, PROD_SHARED_B, false, 1);
+  if (p.splits > 1 && part_bytes < plan_ws_bytes(p, R0, g->C, nph)) p = conv_bwd_plan(g, false);
   if (bnf) {
     TAGI_REQUIRE(nph == 1 && p.splits == 1 && bnf_cfg(p.cfg),
                  "%s: the folded BatchNorm2D backward needs stride 1 and an unsplit one-tile-per-wave plan", what);
@@ -370,19 +377,19 @@ static int conv_bwd_delta_impl(const char* what, const float* dmz, const float* 
     if (add_m) {
       TAGI_REQUIRE(bnf->out_m && bnf->out_S, "%s: null pointer", what);
       if (g->Cout % 16 == 0 && g->k <= 5)
-        return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 3>(a, nph, p, part, part_bytes, s, what, gx);
-      return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 3>(a, nph, p, part, part_bytes, s, what, gx);
+        return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 3, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+      return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 3, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
     }
     if (g->Cout % 16 == 0 && g->k <= 5)
-      return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 1>(a, nph, p, part, part_bytes, s, what, gx);
-    return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 1>(a, nph, p, part, part_bytes, s, what, gx);
+      return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 1, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+    return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 1, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
   }
   if (va && in_place && g->Cout % 16 == 0 && g->k <= 5)
-    return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T>(a, nph, p, part, part_bytes, s, what, gx);
-  if (va && in_place) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4>(a, nph, p, part, part_bytes, s, what, gx);
-  if (va && vb) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B4>(a, nph, p, part, part_bytes, s, what, gx);
-  if (va) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B_S>(a, nph, p, part, part_bytes, s, what, gx);
-  return run_gemm<PROD_SHARED_B, LD_CBWD_A_S, LD_CBWD_B_S>(a, nph, p, part, part_bytes, s, what, gx);
+    return run_gemm<PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 0, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+  if (va && in_place) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 0, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+  if (va && vb) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B4, 0, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+  if (va) return run_gemm<PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B_S, 0, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
+  return run_gemm<PROD_SHARED_B, LD_CBWD_A_S, LD_CBWD_B_S, 0, XD_A>(a, nph, p, part, part_bytes, s, what, gx);
 }
 
 extern "C" int tagi_conv2d_bwd_delta(const float* dmz, const float* dSz, const float* mw, float* dma, float* dSa,
@@ -472,15 +479,16 @@ extern "C" int tagi_conv2d_wgrad(const float* ma, const float* dmz, const float*
   a.Kred = (int)M;
   Plan p = conv_wgrad_plan(g, bias);
   if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, a.R, N, 1)))
-    p = choose_plan(a.R, N, M, 1, PROD_SHARED_A, false, 1);
-  p.tiles_m = (int)cdiv(a.R, kCfg[p.cfg].BM);
+    p = choose_plan(a.R, N, M, 1, PROD_SHARED_A, false, 1, nullptr, XD_B, N < 4);
+  p.tiles_m = (int)cdiv(a.R, cfg_bm(p.cfg, p.xd));
   const bool va = g->C % 4 == 0 && al16(ma);
   const bool vb = g->Cout % 4 == 0 && al16(dmz) && al16(dSz);
   // every 16-pixel run of the reduction inside one image, in whole rows or within one row
   const int64_t howo = g->Ho * g->Wo;
+  a.tile32 = howo % 32 == 0 && (g->Wo % 32 == 0 || 32 % g->Wo == 0);
   if (va && vb && howo % 16 == 0 && (g->Wo % 16 == 0 || 16 % g->Wo == 0))
-    return run_gemm<PROD_SHARED_A, LD_CWG_A4T, LD_STR_MN4>(a, 1, p, ws, ws_bytes, s, what);
-  if (va && vb) return run_gemm<PROD_SHARED_A, LD_CWG_A4, LD_STR_MN4>(a, 1, p, ws, ws_bytes, s, what);
-  if (vb) return run_gemm<PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN4>(a, 1, p, ws, ws_bytes, s, what);
-  return run_gemm<PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN_S>(a, 1, p, ws, ws_bytes, s, what);
+    return run_gemm<PROD_SHARED_A, LD_CWG_A4T, LD_STR_MN4, 0, XD_B>(a, 1, p, ws, ws_bytes, s, what);
+  if (va && vb) return run_gemm<PROD_SHARED_A, LD_CWG_A4, LD_STR_MN4, 0, XD_B>(a, 1, p, ws, ws_bytes, s, what);
+  if (vb) return run_gemm<PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN4, 0, XD_B>(a, 1, p, ws, ws_bytes, s, what);
+  return run_gemm<PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN_S, 0, XD_B>(a, 1, p, ws, ws_bytes, s, what);
 }

@@ -1,5 +1,7 @@
-// fp32-MFMA moment GEMMs for gfx950 (CDNA4): Linear, Conv2D (implicit GEMM on NHWC
-// activations) and the batched attention products all run through one templated kernel.
+// Moment GEMMs for gfx950 (CDNA4): operand loaders, epilogues, planner and launch of Linear,
+// Conv2D (implicit GEMM on NHWC activations) and the batched attention products, and the
+// fp32-MFMA kernel, which runs the batched products and the small Linear and Conv2D ones; the
+// others run the split-operand kernel of tagi_gemm_split.h over the same loaders and epilogues.
 //
 // A TAGI product carries two accumulators per output tile -- the mean and the variance --
 // fed from shared LDS tiles of both operands, with the squared operands formed in
@@ -20,6 +22,7 @@
 // No im2col / col2im buffer exists anywhere.
 #pragma once
 #include <float.h>
+#include <math.h>
 
 #include <type_traits>
 
@@ -51,6 +54,13 @@ enum {
   LD_CFWD_B_S = 13,   // conv fwd weights, scalar (any Cout)
   LD_CBWD_BK4 = 14,   // input-delta weights read in place, w[((c*kk + kh)*kk + kw)*Cout + co]:
                       //   mn = c, k = (ikh,ikw,co), float4 along co (Cout % 4 == 0)
+  // Split kernel only: float4 along rows of any length and alignment (4 bytes). The chunk
+  // that would run past the operand's end is read 1-3 elements earlier and put right, and
+  // elements past the reduction are cleared, by settle() (in the last k tile alone).
+  LD_STR_K4U = 15,    // LD_STR_K4
+  LD_STR_MN4U = 16,   // LD_STR_MN4
+  LD_CFWD_B4U = 22,   // LD_CFWD_B4
+  LD_CBWD_B4U = 23,   // LD_CBWD_B4
   // Tile-aligned conv kinds: the same index maps as LD_CFWD_A4 / LD_CFWD_B4 / LD_CBWD_A4 /
   // LD_CBWD_BK4 / LD_CWG_A4 for geometries where a 16-wide k tile never straddles a kernel
   // tap (C % 16 == 0, or Cout % 16 == 0 for the input delta) or an image (the weight
@@ -70,11 +80,13 @@ struct KindTraits {
   static constexpr bool mn_fast = (KIND == LD_STR_MN4 || KIND == LD_STR_MN_S || KIND == LD_CFWD_B4 ||
                                    KIND == LD_CBWD_B4 || KIND == LD_CBWD_B_S || KIND == LD_CWG_A4 ||
                                    KIND == LD_CWG_A_S || KIND == LD_CFWD_B_S || KIND == LD_CFWD_B4T ||
-                                   KIND == LD_CWG_A4T);
+                                   KIND == LD_CWG_A4T || KIND == LD_STR_MN4U || KIND == LD_CFWD_B4U ||
+                                   KIND == LD_CBWD_B4U);
   static constexpr bool vec4 = (KIND == LD_STR_MN4 || KIND == LD_STR_K4 || KIND == LD_CFWD_A4 || KIND == LD_CFWD_B4 ||
                                 KIND == LD_CBWD_A4 || KIND == LD_CBWD_B4 || KIND == LD_CWG_A4 || KIND == LD_CBWD_BK4 ||
-                                KIND >= LD_CFWD_A4T);
-  static constexpr bool tiled = KIND >= LD_CFWD_A4T;
+                                KIND >= LD_STR_K4U);
+  static constexpr bool tiled = KIND >= LD_CFWD_A4T && KIND <= LD_CWG_A4T;
+  static constexpr bool any = KIND == LD_STR_K4U || KIND == LD_STR_MN4U || KIND == LD_CFWD_B4U || KIND == LD_CBWD_B4U;
 };
 
 // Exact division by an invariant d >= 1 for dividends 0 <= n < 2^31 (Granlund and
@@ -142,8 +154,11 @@ struct Operand {
 // returns zeros (no exec-mask branch and no select per element).
 typedef int tagi_i32x4 __attribute__((ext_vector_type(4)));
 typedef float tagi_f32x4 __attribute__((ext_vector_type(4)));
+typedef float tagi_f32x2 __attribute__((ext_vector_type(2)));
 __device__ tagi_f32x4 tagi_raw_buffer_load_f32x4(tagi_i32x4 rsrc, int voffset, int soffset,
                                                  int aux) __asm("llvm.amdgcn.raw.buffer.load.v4f32");
+__device__ tagi_f32x2 tagi_raw_buffer_load_f32x2(tagi_i32x4 rsrc, int voffset, int soffset,
+                                                 int aux) __asm("llvm.amdgcn.raw.buffer.load.v2f32");
 __device__ float tagi_raw_buffer_load_f32(tagi_i32x4 rsrc, int voffset, int soffset,
                                           int aux) __asm("llvm.amdgcn.raw.buffer.load.f32");
 
@@ -232,6 +247,7 @@ struct GemmArgs {
   int tiles_m, tiles_n;
   int splits, k_chunk;
   int phased;      // conv input delta: z indexes the stride phase
+  int tile32;      // conv kinds: 32-wide k tiles stay within a kernel tap (or an image)
   float* partial;  // split-K partial sums, or null to apply the epilogue in place
   // phased launches: blockIdx.y / splits -> phase, longest reductions first so the short
   // phases fill in behind them
@@ -240,10 +256,24 @@ struct GemmArgs {
 
 template <int BM_, int BN_, int WM_, int WN_>
 struct Cfg {
+  static constexpr bool X = false;
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = 16;
   static constexpr int NTH = (BM / WM) * (BN / WN) * 64;
   // blocks per CU the register budget is sized for (2 x 256-thread blocks = 2 waves/SIMD)
   static constexpr int MINB = NTH >= 512 ? 1 : 2;
+};
+
+// Tile of the split-operand kernel (tagi_gemm_split.h): NW waves, each with DM rows of the
+// operand read straight into registers and all LM rows of the one staged through LDS, whose
+// tiles are held in NBUF LDS buffers; MINW: waves per SIMD the register budget is sized for.
+// F: the forward product's values, S: the two-product kernels'.
+template <int NW_, int DM_, int LM_, int NBUF_F, int MINW_F, int NBUF_S, int MINW_S>
+struct XCfg {
+  static constexpr bool X = true;
+  static constexpr int NW = NW_, DM = DM_, LM = LM_, BK = 32;
+  static constexpr int NTH = 64 * NW;
+  static constexpr int nbuf(int prod) { return prod == PROD_FWD ? NBUF_F : NBUF_S; }
+  static constexpr int minw(int prod) { return prod == PROD_FWD ? MINW_F : MINW_S; }
 };
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I = B .. E-1, in order.
@@ -260,17 +290,41 @@ __device__ __forceinline__ void static_for(F&& f) {
 // the chunk -> (mn, k) map is fixed per thread, so per-row / per-k invariants are
 // computed once in init().
 // ------------------------------------------------------------------------------------
-template <int KIND, int NT, int BMN, int BK, int NTH, int PF = 1>
+// MAP says which chunks a thread owns:
+//   0  consecutive chunks of the tile (the fp32 kernel's LDS stores)
+//   1  units whose elements are consecutive along the reduction, so that a unit's bf16
+//      parts are written to LDS packed (the split kernel's staged operand): 8 k of one row,
+//      or KG k of 4 rows where the float4 run along the tile dim
+//   2  MFMA fragments: 16 rows of DMN per fragment, lane l the row l % 16 and
+//      k = 8 (l / 16) .. + 7 (the split kernel's direct operand; wave w owns rows w DMN ..)
+template <int KIND, int NT, int BMN, int BK, int NTH, int PF = 1, int MAP = 0, int DMN = 0>
 struct Loader {
   static constexpr bool V4 = KindTraits<KIND>::vec4;
   static constexpr bool MNF = KindTraits<KIND>::mn_fast;
-  static constexpr int W = V4 ? 4 : 1;  // elements per chunk
+  // elements per chunk: a float4; MAP 1 along the tile dim, a float2 where float4 units of
+  // two k would leave threads without one; MAP 2 along the tile dim, one element of each of
+  // the DMN / 16 fragments (which take every (DMN / 16)-th row), so that one load serves all
+  static constexpr int FV = (MAP == 2 && V4 && MNF) ? DMN / 16 : 0;
+  static_assert(FV == 0 || FV == 1 || FV == 2, "one or two fragments per load");
+  static constexpr bool HALF = MAP == 1 && V4 && MNF && BMN * BK / 4 < 2 * NTH;
+  static constexpr int W = !V4 ? 1 : FV ? FV : HALF ? 2 : 4;
   static constexpr int NCH = BMN * BK / W;  // chunks in the tile
+  // MAP 1: rows per unit, k per unit (a power of two, 2 to 8), units in the tile; MAP 2:
+  // chunks per fragment and lane
+  static constexpr int UR = (V4 && MNF) ? W : 1;
+  static constexpr int KG0 = BMN * BK / UR / NTH;
+  static constexpr int KG = MAP != 1 || KG0 >= 8 ? 8 : (V4 && !MNF) ? 4 : KG0;
+  static_assert(MAP != 1 || (KG >= 2 && (KG & (KG - 1)) == 0), "units hold 2, 4 or 8 consecutive k");
+  static constexpr int NUNIT = (BMN / UR) * (BK / KG);
+  static constexpr int CPU = KG * UR / W;
+  static constexpr int NU = NUNIT / NTH;
+  static constexpr int CPF = 8 / ((V4 && !MNF) ? 4 : 1);
   // fewer chunks than threads (a 32-wide operand of a 4-wave block): threads past NCH idle
-  static constexpr bool PART = NCH < NTH;
-  static constexpr int NC = PART ? 1 : NCH / NTH;
-  static_assert(PART ? (NCH * W == BMN * BK && NTH % NCH == 0) : (NC * W * NTH == BMN * BK),
+  static constexpr bool PART = MAP == 0 && NCH < NTH;
+  static constexpr int NC = MAP == 0 ? (PART ? 1 : NCH / NTH) : (MAP == 1 ? NU * CPU : FV ? 8 : DMN / 16 * CPF);
+  static_assert(MAP != 0 || (PART ? (NCH * W == BMN * BK && NTH % NCH == 0) : (NC * W * NTH == BMN * BK)),
                 "tile does not split evenly over threads");
+  static_assert(MAP != 1 || NU * NTH == NUNIT, "units do not split evenly over threads");
   static constexpr int LD = BMN + 4;
   // LDS tile of one tensor. Reduction-major [BK][LD] (rows of the tile dim padded by 4),
   // except for float4 loaders that walk the reduction ("K4" kinds): those keep the tile
@@ -282,29 +336,40 @@ struct Loader {
   // the fragment reads (one row per lane).
   static constexpr bool KMAJ = V4 && !MNF;
   static constexpr int TILE = KMAJ ? BMN * BK : BK * LD;
-  static_assert(!KMAJ || BK == 16, "the row-major tile swizzle assumes 4 chunks per row");
+  static_assert(MAP != 0 || !KMAJ || BK == 16, "the row-major tile swizzle assumes 4 chunks per row");
   __device__ static __forceinline__ int kmaj_off(int row, int k) {
     return row * BK + ((((k >> 2) ^ (row >> 1) ^ (row >> 2)) & 3) << 2);
   }
 
-  using Vt = typename std::conditional<V4, float4, float>::type;
-  static constexpr bool CONV_ROWS = (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S || KIND == LD_CBWD_A4 ||
+  using Vt = typename std::conditional<W == 4, float4, typename std::conditional<W == 2, float2, float>::type>::type;
+  static constexpr bool CONV_ROWS = MAP != 2 && (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S || KIND == LD_CBWD_A4 ||
                                      KIND == LD_CBWD_A_S);
   static constexpr bool CONV_R = CONV_ROWS || KIND == LD_CBWD_B4 || KIND == LD_CBWD_B_S || KIND == LD_CBWD_BK4 ||
-                                 KIND == LD_CWG_A4 || KIND == LD_CWG_A_S;
+                                 KIND == LD_CWG_A4 || KIND == LD_CWG_A_S || KIND == LD_CBWD_B4U;
   static constexpr int NRB = CONV_ROWS ? NC : 1;  // per-chunk row bases only where rows differ
   static constexpr int NR = CONV_R ? NC : 1;
 
+  static constexpr bool TILED0 = KindTraits<KIND>::tiled;
   Vt v[PF][NT][NC];  // PF register stages of fetched chunks
   // kinds with a ones row (the bias sums of a parameter-delta product): the chunk holds
   // that row, whose first element is written as 1.0 when the chunk is stored to LDS (a
   // select on the loaded value at fetch time would wait for the load right there)
   static constexpr bool ONES = (KIND == LD_STR_MN4 || KIND == LD_STR_MN_S || KIND == LD_STR_K_S ||
-                                KIND == LD_CWG_A4 || KIND == LD_CWG_A_S || KIND == LD_CWG_A4T);
-  static constexpr bool TILED = KindTraits<KIND>::tiled;
+                                KIND == LD_CWG_A4 || KIND == LD_CWG_A_S || KIND == LD_CWG_A4T ||
+                                (KIND == LD_STR_MN4U && MAP == 1));
+  static constexpr bool ANY = KindTraits<KIND>::any;
+  // conv patches as MFMA fragments: a lane's k values are decoded once for all its
+  // fragments (each row keeps its base offset and tap mask in lb / tapm; kk <= 5)
+  static constexpr bool PATCH = MAP == 2 && (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S || KIND == LD_CBWD_A4 ||
+                                             KIND == LD_CBWD_A_S);
+  static constexpr int NLB = TILED0 ? NC : PATCH ? DMN / 16 : 1;
+  static constexpr bool TILED = TILED0;
   bool onef[ONES ? PF : 1][ONES ? NC : 1];
+  int onep[ONES && ANY ? NC : 1];  // where in its chunk the ones row lies (kinds of any alignment)
   FastDiv dnkw;              // divider for the phase's taps per row (conv input delta)
   int mnmax, kmax;           // extents checked by fetch (per phase for the conv input delta)
+  int kfull;                 // the whole reduction (kmax ends with the block's stretch of it)
+  uint32_t nel;              // the operand's elements
   int cmn[NC], ck[NC];       // chunk origin within the tile
   bool active;               // this thread loads a chunk (always, unless PART)
   int rowbase[NRB];          // per-chunk image base (conv rows), elements from the operand base
@@ -313,13 +378,48 @@ struct Loader {
   // tile-aligned kinds: per-chunk byte offset of the chunk at the tile's origin (modulo
   // 2^32; the tile's scalar part is added per fetch), tap masks, and the weight delta's
   // input-row / input-column offsets of the chunk's pixel and kernel tap
-  uint32_t lb[TILED ? NC : 1], tapm[TILED ? NC : 1];
+  uint32_t lb[NLB], tapm[NLB];
   int lih[TILED ? NC : 1], liw[TILED ? NC : 1];
   bool okl[TILED ? NC : 1], onel[TILED ? NC : 1];
   int tkh0, tkw0, tnkw;      // input delta: the phase's first tap and taps per row
   uint32_t oobv;             // kBufOutOfRange, held in a register
 
+  // MAP 1: first row and first k of the thread's unit u
+  __device__ static __forceinline__ void unit_pos(int tid, int u, int& mn, int& k) {
+    const int x = tid + u * NTH;
+    if constexpr (!V4 && MNF) {  // scalar, rows consecutive over the lanes
+      mn = x % BMN;
+      k = (x / BMN) * KG;
+    } else {
+      mn = x / (BK / KG) * UR;
+      k = (x % (BK / KG)) * KG;
+    }
+  }
+
   __device__ __forceinline__ void map(int tid) {
+    if constexpr (MAP == 1) {
+      active = true;
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        int mn, k;
+        unit_pos(tid, u, mn, k);
+#pragma unroll
+        for (int c = 0; c < CPU; ++c) {
+          cmn[u * CPU + c] = mn;
+          ck[u * CPU + c] = k + ((V4 && !MNF) ? 4 * c : c);
+        }
+      }
+      return;
+    }
+    if constexpr (MAP == 2) {
+      active = true;
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        cmn[i] = (tid >> 6) * DMN + (FV ? FV * (tid & 15) : (i / CPF) * 16 + (tid & 15));
+        ck[i] = 8 * ((tid & 63) >> 4) + (FV ? i : (i % CPF) * W);
+      }
+      return;
+    }
     active = !PART || tid < NCH;
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
@@ -342,7 +442,7 @@ struct Loader {
     mnmax = o.MN;
     kmax = o.K;
     if constexpr (KIND == LD_CBWD_A4 || KIND == LD_CBWD_A_S || KIND == LD_CBWD_B4 || KIND == LD_CBWD_B_S ||
-                  KIND == LD_CBWD_BK4 || KIND == LD_CBWD_A4T || KIND == LD_CBWD_BK4T) {
+                  KIND == LD_CBWD_BK4 || KIND == LD_CBWD_A4T || KIND == LD_CBWD_BK4T || KIND == LD_CBWD_B4U) {
       const Phase ph = make_phase(o.g, z);
       kmax = ph.nkh * ph.nkw * o.g.Cout;
       dnkw = make_fastdiv(ph.nkw > 0 ? ph.nkw : 1);
@@ -351,11 +451,14 @@ struct Loader {
       tkw0 = ph.kw0;
       tnkw = ph.nkw;
     }
-    kmax = min(kmax, klim);
     oobv = kBufOutOfRange;
     asm volatile("" : "+v"(oobv));  // one register for every chunk's out-of-range offset
+    kfull = kmax;
+    kmax = min(kmax, klim);
     if constexpr (TILED) init_tiled(o, z, mn0);
-    if constexpr (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S) {
+    if constexpr (PATCH) {
+      init_patch(o, z, mn0);
+    } else if constexpr (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S) {
       // rows are output pixels: base of image n and the top-left input corner
       const int howo = o.g.Ho * o.g.Wo;
 #pragma unroll
@@ -394,7 +497,7 @@ struct Loader {
         }
         r2[i] = ph.nkw;
       }
-    } else if constexpr (KIND == LD_CBWD_B4 || KIND == LD_CBWD_B_S || KIND == LD_CBWD_BK4) {
+    } else if constexpr (KIND == LD_CBWD_B4 || KIND == LD_CBWD_B_S || KIND == LD_CBWD_BK4 || KIND == LD_CBWD_B4U) {
       // tap offsets of this phase
       const Phase ph = make_phase(o.g, z);
 #pragma unroll
@@ -416,7 +519,12 @@ struct Loader {
         r2[i] = c;
       }
     }
-    if constexpr (CONV_R || TILED || KIND == LD_CFWD_B4 || KIND == LD_CFWD_B_S) {
+    nel = (uint32_t)(o.nbytes >> 2);
+    if constexpr (ONES && ANY) {
+#pragma unroll
+      for (int i = 0; i < NC; ++i) onep[i] = o.ones_row - mn0 - cmn[i];
+    }
+    if constexpr (CONV_R || PATCH || TILED || KIND == LD_CFWD_B4 || KIND == LD_CFWD_B_S || KIND == LD_CFWD_B4U) {
       rs0 = make_buffer_rsrc(o.p0, o.nbytes);
       rs1 = make_buffer_rsrc(NT == 2 ? o.p1 : o.p0, o.nbytes);
     } else {
@@ -441,6 +549,49 @@ struct Loader {
     return m;
   }
 
+  // Output pixel mn (conv forward): element offset of its top-left input corner (modulo
+  // 2^32) and the mask of the taps inside the image
+  __device__ __forceinline__ void fwd_row(const Operand& o, int mn, uint32_t& base, uint32_t& msk) const {
+    using U = uint32_t;
+    const ConvG& g = o.g;
+    base = msk = 0;
+    if (mn < o.MN) {
+      const int howo = g.Ho * g.Wo;
+      const int n = mn / howo, p = mn - n * howo;
+      const int oh = p / g.Wo, ow = p - oh * g.Wo;
+      const int ih0 = oh * g.stride - g.pt, iw0 = ow * g.stride - g.pl;
+      base = ((U(n) * U(g.H) + U(ih0)) * U(g.W) + U(iw0)) * U(g.C);
+      msk = spread_bits(range_bits(-ih0, g.H - ih0, g.kk), range_bits(-iw0, g.W - iw0, g.kk), g.kk, g.kk);
+    }
+  }
+  // Input pixel mn of stride phase z (conv input delta): element offset of the output pixel
+  // that tap (kh0, kw0) takes it to, and the mask of the phase's taps inside the output
+  __device__ __forceinline__ void bwd_row(const Operand& o, int z, int mn, uint32_t& base, uint32_t& msk) const {
+    using U = uint32_t;
+    const ConvG& g = o.g;
+    const Phase ph = make_phase(g, z);
+    const int hq = ph.Hq * ph.Wq;
+    base = msk = 0;
+    if (mn < mnmax && hq > 0) {
+      const int n = mn / hq, rr = mn - n * hq;
+      const int hh = rr / ph.Wq, ww = rr - hh * ph.Wq;
+      const int h = hh * g.stride + ph.a, w = ww * g.stride + ph.b;
+      const int r0 = (h + g.pt - ph.kh0) / g.stride, r1 = (w + g.pl - ph.kw0) / g.stride;
+      base = ((U(n) * U(g.Ho) + U(r0)) * U(g.Wo) + U(r1)) * U(g.Cout);
+      // output row r0 - ikh in [0, Ho) and column r1 - ikw in [0, Wo)
+      msk = spread_bits(range_bits(r0 - g.Ho + 1, r0 + 1, ph.nkh), range_bits(r1 - g.Wo + 1, r1 + 1, ph.nkw), ph.nkh,
+                        ph.nkw);
+    }
+  }
+
+  __device__ __forceinline__ void init_patch(const Operand& o, int z, int mn0) {
+#pragma unroll
+    for (int f = 0; f < NLB; ++f) {
+      if constexpr (KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S) fwd_row(o, mn0 + cmn[f * CPF], lb[f], tapm[f]);
+      else bwd_row(o, z, mn0 + cmn[f * CPF], lb[f], tapm[f]);
+    }
+  }
+
   __device__ __forceinline__ void init_tiled(const Operand& o, int z, int mn0) {
     using U = uint32_t;
     const ConvG& g = o.g;
@@ -448,49 +599,27 @@ struct Loader {
     for (int i = 0; i < NC; ++i) {
       const int mn = mn0 + cmn[i];
       if constexpr (KIND == LD_CFWD_A4T) {
-        // row = output pixel (n, oh, ow); chunk = 4 channels at k offset ck of tap (kh, kw)
-        uint32_t base = 0, msk = 0;
-        if (mn < o.MN) {
-          const int howo = g.Ho * g.Wo;
-          const int n = mn / howo, p = mn - n * howo;
-          const int oh = p / g.Wo, ow = p - oh * g.Wo;
-          const int ih0 = oh * g.stride - g.pt, iw0 = ow * g.stride - g.pl;
-          base = ((U(n) * U(g.H) + U(ih0)) * U(g.W) + U(iw0)) * U(g.C) + U(ck[i]);
-          msk = spread_bits(range_bits(-ih0, g.H - ih0, g.kk), range_bits(-iw0, g.W - iw0, g.kk), g.kk, g.kk);
-        }
-        lb[i] = base * 4u;
-        tapm[i] = msk;
+        // row = output pixel; chunk = 4 channels at k offset ck of a tap
+        fwd_row(o, mn, lb[i], tapm[i]);
+        lb[i] = (lb[i] + U(ck[i])) * 4u;
       } else if constexpr (KIND == LD_CFWD_B4T) {
         // weights w[(c*kk2 + kidx)*Cout + co]: chunk = 4 co at reduction offset ck (channel c0 + ck)
         lb[i] = (U(ck[i]) * U(g.kk * g.kk) * U(g.Cout) + U(mn)) * 4u;
         okl[i] = mn < o.MN;
       } else if constexpr (KIND == LD_CBWD_A4T) {
-        // row = input pixel of stride phase z; (r0, r1) = output pixel of tap (kh0, kw0)
-        const Phase ph = make_phase(g, z);
-        const int hq = ph.Hq * ph.Wq;
-        uint32_t base = 0, msk = 0;
-        if (mn < mnmax && hq > 0) {
-          const int n = mn / hq, rr = mn - n * hq;
-          const int hh = rr / ph.Wq, ww = rr - hh * ph.Wq;
-          const int h = hh * g.stride + ph.a, w = ww * g.stride + ph.b;
-          const int r0 = (h + g.pt - ph.kh0) / g.stride, r1 = (w + g.pl - ph.kw0) / g.stride;
-          base = ((U(n) * U(g.Ho) + U(r0)) * U(g.Wo) + U(r1)) * U(g.Cout) + U(ck[i]);
-          // output row r0 - ikh in [0, Ho) and column r1 - ikw in [0, Wo)
-          msk = spread_bits(range_bits(r0 - g.Ho + 1, r0 + 1, ph.nkh), range_bits(r1 - g.Wo + 1, r1 + 1, ph.nkw),
-                            ph.nkh, ph.nkw);
-        }
-        lb[i] = base * 4u;
-        tapm[i] = msk;
+        // row = input pixel of stride phase z; chunk = 4 co at k offset ck of a tap
+        bwd_row(o, z, mn, lb[i], tapm[i]);
+        lb[i] = (lb[i] + U(ck[i])) * 4u;
       } else if constexpr (KIND == LD_CBWD_BK4T) {
         // weights w[((c*kk + kh)*kk + kw)*Cout + co] in place: row c, chunk = 4 co at offset ck
         lb[i] = (U(mn) * U(g.kk * g.kk) * U(g.Cout) + U(ck[i])) * 4u;
         okl[i] = mn < mnmax;
       } else if constexpr (KIND == LD_CWG_A4T) {
         // row = weight row (kh, kw, c) (+ the ones row); the chunk's pixel is at offset ck
-        // of a 16-pixel run inside one image, (dh, dw) rows/columns past the run's start
+        // of a BK-pixel run inside one image, (dh, dw) rows/columns past the run's start
         const int kidx = mn / g.C, c = mn - kidx * g.C;
         const int kh = kidx / g.kk, kw = kidx - kh * g.kk;
-        const int dh = g.Wo >= 16 ? 0 : ck[i] / g.Wo, dw = ck[i] - dh * g.Wo;
+        const int dh = g.Wo >= BK ? 0 : ck[i] / g.Wo, dw = ck[i] - dh * g.Wo;
         int ih = dh * g.stride - g.pt + kh;
         const int iw = dw * g.stride - g.pl + kw;
         if (mn >= o.MN) ih = -(1 << 28);  // past the weight rows: reads zeros
@@ -502,28 +631,32 @@ struct Loader {
     }
   }
 
-  template <int ST>
+  // TT: the tensor to load (-1: all)
+  template <int ST, int TT>
   __device__ __forceinline__ void load_chunk(int i, uint32_t vo) {
-    if constexpr (V4) {
-      const tagi_f32x4 a = tagi_raw_buffer_load_f32x4(rs0, (int)vo, 0, 0);
-      v[ST][0][i] = make_float4(a.x, a.y, a.z, a.w);
-      if constexpr (NT == 2) {
-        const tagi_f32x4 b = tagi_raw_buffer_load_f32x4(rs1, (int)vo, 0, 0);
-        v[ST][1][i] = make_float4(b.x, b.y, b.z, b.w);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (TT >= 0 && t != TT) continue;
+      const tagi_i32x4 rs = t == 0 ? rs0 : rs1;
+      if constexpr (W == 2) {
+        const tagi_f32x2 a = tagi_raw_buffer_load_f32x2(rs, (int)vo, 0, 0);
+        v[ST][t][i] = make_float2(a.x, a.y);
+      } else if constexpr (W == 4) {
+        const tagi_f32x4 a = tagi_raw_buffer_load_f32x4(rs, (int)vo, 0, 0);
+        v[ST][t][i] = make_float4(a.x, a.y, a.z, a.w);
+      } else {
+        v[ST][t][i] = tagi_raw_buffer_load_f32(rs, (int)vo, 0, 0);
       }
-    } else {
-      v[ST][0][i] = tagi_raw_buffer_load_f32(rs0, (int)vo, 0, 0);
-      if constexpr (NT == 2) v[ST][1][i] = tagi_raw_buffer_load_f32(rs1, (int)vo, 0, 0);
     }
   }
 
   // Tile-aligned kinds: the tile's tap / pixel run is decoded in scalar registers
   // (k0 is the same for every lane), then one add and a mask bit per chunk.
-  template <int ST>
+  template <int ST, int TT>
   __device__ __forceinline__ void fetch_tiled(const Operand& o, int k0) {
     using U = uint32_t;
     const ConvG& g = o.g;
-    const bool kin = k0 < kmax;  // whole tile in range (the reduction length is a multiple of 16)
+    const bool kin = k0 < kmax;  // whole tile in range (the reduction length is a multiple of BK)
     if constexpr (KIND == LD_CFWD_A4T || KIND == LD_CFWD_B4T) {
       const int kidx = fdiv(k0, g.dC), c0 = k0 - kidx * g.C;
       if constexpr (KIND == LD_CFWD_A4T) {
@@ -532,12 +665,12 @@ struct Loader {
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
           const bool ok = kin && ((tapm[i] >> (kidx & 31)) & 1u);
-          load_chunk<ST>(i, ok ? lb[i] + s4 : oobv);
+          load_chunk<ST, TT>(i, ok ? lb[i] + s4 : oobv);
         }
       } else {
         const uint32_t s4 = (U(c0) * U(g.kk * g.kk) + U(kidx)) * U(g.Cout) * 4u;
 #pragma unroll
-        for (int i = 0; i < NC; ++i) load_chunk<ST>(i, (kin && okl[i]) ? lb[i] + s4 : oobv);
+        for (int i = 0; i < NC; ++i) load_chunk<ST, TT>(i, (kin && okl[i]) ? lb[i] + s4 : oobv);
       }
     } else if constexpr (KIND == LD_CBWD_A4T || KIND == LD_CBWD_BK4T) {
       const int kidx = fdiv(k0, g.dCout), co0 = k0 - kidx * g.Cout;
@@ -547,13 +680,13 @@ struct Loader {
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
           const bool ok = kin && ((tapm[i] >> (kidx & 31)) & 1u);
-          load_chunk<ST>(i, ok ? lb[i] - s4 : oobv);
+          load_chunk<ST, TT>(i, ok ? lb[i] - s4 : oobv);
         }
       } else {
         const int kh = tkh0 + ikh * g.stride, kw = tkw0 + ikw * g.stride;
         const uint32_t s4 = ((U(kh) * U(g.kk) + U(kw)) * U(g.Cout) + U(co0)) * 4u;
 #pragma unroll
-        for (int i = 0; i < NC; ++i) load_chunk<ST>(i, (kin && okl[i]) ? lb[i] + s4 : oobv);
+        for (int i = 0; i < NC; ++i) load_chunk<ST, TT>(i, (kin && okl[i]) ? lb[i] + s4 : oobv);
       }
     } else if constexpr (KIND == LD_CWG_A4T) {
       const int n = fdiv(k0, g.dHW), p0 = k0 - n * (g.Ho * g.Wo);
@@ -565,20 +698,119 @@ struct Loader {
         const int ih = sih + lih[i], iw = siw + liw[i];
         const bool ok = kin && U(ih) < U(g.H) && U(iw) < U(g.W);
         onef[ST][i] = kin && onel[i];
-        load_chunk<ST>(i, ok ? lb[i] + s4 : oobv);
+        load_chunk<ST, TT>(i, ok ? lb[i] + s4 : oobv);
       }
+    }
+  }
+
+  // Conv patch fragments: the lane's 8 k values (two float4 chunks, or 8 elements) are decoded
+  // to an offset and a tap once, then each of its rows adds its base and tests its mask.
+  template <int ST, int TT>
+  __device__ __forceinline__ void fetch_patch(const Operand& o, int k0) {
+    using U = uint32_t;
+    const ConvG& g = o.g;
+    constexpr bool FWD = KIND == LD_CFWD_A4 || KIND == LD_CFWD_A_S;
+    const int run = FWD ? g.C : g.Cout;  // elements of one tap
+    const int ntw = FWD ? g.kk : tnkw;   // taps per kernel row
+    int k = k0 + ck[0];
+    int tap = fdiv(k, FWD ? g.dC : g.dCout), c = k - tap * run;
+    const int th0 = fdiv(tap, FWD ? g.dkk : dnkw);
+    int th = th0, tw = tap - th * ntw;
+    uint32_t d[CPF];
+    int tp[CPF];
+#pragma unroll
+    for (int e = 0; e < CPF; ++e) {
+      tp[e] = k < kmax ? tap : 31;  // no tap has index 31
+      if constexpr (FWD) d[e] = (U(th) * U(g.W) + U(tw)) * U(run) + U(c);
+      else d[e] = U(c) - (U(th) * U(g.Wo) + U(tw)) * U(run);
+      if (e + 1 < CPF) {
+        k += W;
+        c += W;
+        // (a run can be shorter than the step only for scalar chunks, where the step is 1)
+        const bool nt = c >= run;
+        c = nt ? c - run : c;
+        tap += nt;
+        tw += nt;
+        const bool nr = tw >= ntw;
+        tw = nr ? 0 : tw;
+        th += nr;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NC; ++i) {
+      const int f = i / CPF, e = i % CPF;
+      const bool ok = (tapm[f] >> tp[e]) & 1u;
+      load_chunk<ST, TT>(i, ok ? (lb[f] + d[e]) * 4u : oobv);
     }
   }
 
   // Gather of one k tile: each chunk's reduction index is decoded with exact
   // multiply-high divisions; chunks outside the operand or in the zero padding read as 0.
-  template <int ST = 0>
+  // Kinds of any alignment: element offset of chunk i at (mn, k), and whether it is read
+  __device__ __forceinline__ bool locate(const Operand& o, int mn, int k, int i, uint32_t& off) const {
+    using U = uint32_t;
+    if constexpr (KIND == LD_STR_K4U) {
+      off = U(mn) * U(o.s_mn) + U(k);
+    } else if constexpr (KIND == LD_STR_MN4U) {
+      off = U(mn) + U(k) * U(o.s_k);
+    } else if constexpr (KIND == LD_CFWD_B4U) {
+      const int kidx = fdiv(k, o.g.dC), c = k - kidx * o.g.C;
+      off = (U(c) * U(o.g.kk * o.g.kk) + U(kidx)) * U(o.g.Cout) + U(mn);
+    } else {
+      const int kidx = fdiv(k, o.g.dCout), co = k - kidx * o.g.Cout;
+      const int ikh = fdiv(kidx, dnkw), ikw = kidx - ikh * tnkw;
+      off = ((U(tkh0 + ikh * o.g.stride) * U(o.g.kk) + U(tkw0 + ikw * o.g.stride)) * U(o.g.Cout) + U(co)) * U(o.g.C) +
+            U(mn);
+    }
+    return k < kmax && mn < mnmax;
+  }
+
+  // After the loads of k tile k0 (kinds of any alignment): the shifted chunk at the operand's
+  // end, which the last tile of the reduction holds, and elements past the reduction.
+  // Rows past the tile dim hold other rows' values: they reach no stored output.
+  __device__ __forceinline__ void settle(const Operand& o, int mn0, int k0) {
+    if constexpr (ANY) {
+      if (k0 + BK >= kfull) {
+        constexpr int CW = W;
+        static_for<0, NC>([&](auto I) {
+          constexpr int i = decltype(I)::value;
+          const int mn = mn0 + cmn[i], k = k0 + ck[i];
+          uint32_t off = 0;
+          const bool ok = locate(o, mn, k, i, off);
+          const uint32_t last = nel - CW;
+          const int sh = ok && off > last ? (int)(off - last) : 0;
+          const int keep = KIND == LD_STR_K4U ? kmax - k : CW;  // elements within the reduction
+          static_for<0, NT>([&](auto T) {
+            Vt& c = v[0][decltype(T)::value][i];
+            if constexpr (CW == 2) {
+              if (sh) c.x = c.y;
+            } else if constexpr (CW == 4) {
+              const float x0 = c.x, x1 = c.y, x2 = c.z, x3 = c.w;
+              const float y0 = sh == 0 ? x0 : sh == 1 ? x1 : sh == 2 ? x2 : x3;
+              const float y1 = sh == 0 ? x1 : sh == 1 ? x2 : x3;
+              const float y2 = sh == 0 ? x2 : x3;
+              c.x = keep > 0 ? y0 : 0.f;
+              c.y = keep > 1 ? y1 : 0.f;
+              c.z = keep > 2 ? y2 : 0.f;
+              c.w = keep > 3 ? x3 : 0.f;
+            }
+          });
+        });
+      }
+    }
+  }
+
+  template <int ST = 0, int TT = -1>
   __device__ __forceinline__ void fetch(const Operand& o, int z, int mn0, int k0) {
     if constexpr (PART) {
       if (!active) return;
     }
     if constexpr (TILED) {
-      fetch_tiled<ST>(o, k0);
+      fetch_tiled<ST, TT>(o, k0);
+      return;
+    }
+    if constexpr (PATCH) {
+      fetch_patch<ST, TT>(o, k0);
       return;
     }
 #pragma unroll
@@ -590,7 +822,12 @@ struct Loader {
       // in unsigned arithmetic because chunks that are not ok may compute anything
       uint32_t off = 0;
       using U = uint32_t;
-      if constexpr (KIND == LD_STR_MN4 || KIND == LD_STR_MN_S || KIND == LD_STR_K_S) {
+      if constexpr (ANY) {
+        ok = locate(o, mn, k, i, off);
+        if constexpr (ONES) one = k < kmax && o.ones_row >= mn && o.ones_row < mn + W;
+        const uint32_t last = nel - W;
+        off = off < last ? off : last;
+      } else if constexpr (KIND == LD_STR_MN4 || KIND == LD_STR_MN_S || KIND == LD_STR_K_S) {
         ok = k < kmax && mn < o.MN;
         one = k < kmax && mn == o.ones_row;
         if constexpr (KIND == LD_STR_MN4) off = U(mn) + U(k) * U(o.s_k);
@@ -645,8 +882,21 @@ struct Loader {
       }
       if constexpr (ONES) onef[ST][i] = one;
       (void)one;
-      load_chunk<ST>(i, ok ? off * 4u : oobv);
+      load_chunk<ST, TT>(i, ok ? off * 4u : oobv);
     }
+  }
+
+  // MAP 1 and 2: element e of chunk i of tensor t
+  template <int ST = 0>
+  __device__ __forceinline__ float elem(int t, int i, int e) const {
+    float x;
+    if constexpr (W == 2) x = e == 0 ? v[ST][t][i].x : v[ST][t][i].y;
+    else if constexpr (W == 4) x = e == 0 ? v[ST][t][i].x : e == 1 ? v[ST][t][i].y : e == 2 ? v[ST][t][i].z : v[ST][t][i].w;
+    else x = v[ST][t][i];
+    if constexpr (ONES) {
+      if (t == 0 && (ANY ? e == onep[ANY ? i : 0] : e == 0) && onef[ST][i]) x = 1.f;
+    }
+    return x;
   }
 
   template <int ST = 0>
@@ -875,6 +1125,565 @@ __device__ __forceinline__ int kred_of(const GemmArgs& g, int z) {
   return ph.nkh * ph.nkw * g.a.g.Cout;
 }
 
+// The tile, split and stretch of the reduction a block works on; false for a block past its
+// phase's tiles.
+struct BlockPos {
+  int z, split, R, tmi, m0, n0, kbeg, kend;
+};
+
+template <int BM, int BN>
+__device__ __forceinline__ bool block_pos(const GemmArgs& g, BlockPos& p) {
+  // Split-K launches with at least 8 split groups: every tile of one split group (the
+  // tiles that read the same stretch of the reduction) goes to one XCD. Workgroups are
+  // dealt round-robin over the 8 XCDs in linear-id order, so the linear id L is read as
+  // (XCD x = L mod 8, k-th block of that XCD) and group 8*(k / nt) + x, tile k mod nt
+  // are assigned; groups past the last multiple of 8 keep the plain order. Without this,
+  // the tiles of a group land on different XCDs and each XCD's L2 fetches the shared
+  // operand panels again (the parameter-delta GEMMs' 9 tap tiles share one pixel range).
+  int zq, bid;
+  bool xcd_tiles = true;
+  if (!g.phased && g.splits > 1 && gridDim.y >= 8 && (uint64_t)gridDim.x * gridDim.y < (1ull << 31)) {
+    const int nt0 = g.tiles_m * g.tiles_n;
+    const int L = blockIdx.x + blockIdx.y * gridDim.x;
+    const int g8 = (int)(gridDim.y & ~7u);
+    int grp, tile;
+    if (L < g8 * nt0) {
+      const int k = L >> 3, q = k / nt0;
+      grp = q * 8 + (L & 7);
+      tile = k - q * nt0;
+    } else {
+      const int L2 = L - g8 * nt0, q = L2 / nt0;
+      grp = g8 + q;
+      tile = L2 - q * nt0;
+    }
+    zq = grp / g.splits;
+    p.split = grp - zq * g.splits;
+    bid = tile;
+    xcd_tiles = false;
+  } else {
+    zq = blockIdx.y / g.splits;
+    p.split = blockIdx.y - zq * g.splits;
+    bid = blockIdx.x;
+  }
+  const int z = g.phased ? (int)g.phase_order[zq] : zq;
+  p.z = z;
+  p.R = rows_of(g, z);
+  const int Kred = kred_of(g, z);
+  const int tiles_m = g.phased ? (p.R + BM - 1) / BM : g.tiles_m;
+
+  // XCD-aware tile order: workgroups are dealt round-robin over the 8 XCDs, so map
+  // consecutive block ids of one XCD onto consecutive tiles (shared operand panels stay
+  // in that XCD's L2).
+  const int nt = tiles_m * g.tiles_n;
+  if (bid >= nt) return false;  // phased launches size the grid for the largest phase
+  const int per = nt >> 3;
+  const int t = (xcd_tiles && bid < (per << 3)) ? ((bid & 7) * per + (bid >> 3)) : bid;
+  p.tmi = t / g.tiles_n;
+  p.m0 = p.tmi * BM;
+  p.n0 = (t - p.tmi * g.tiles_n) * BN;
+  p.kbeg = p.split * g.k_chunk;
+  p.kend = min(Kred, p.kbeg + g.k_chunk);
+  return true;
+}
+
+// The epilogue of one block tile: split-K partial sums, or the layer's epilogue. FR: the
+// MFMA's rows and columns (32, or 16 in the split-operand kernels); lane l holds column
+// l % FR of its wave's FR x FR tiles, in rows 8 (v / 4) + 4 (l / FR) + v % 4 (CI: tile j's
+// columns are every TN-th column of the wave's, from j on). EK: the epilogue kinds the
+// caller launches, one bit each. SMEM: the floats of LDS the caller holds, free to be overwritten here. epf_s / epb_h / epb_j: the
+// operands the EPF / EPFB kernels loaded during their last k-period.
+template <int FR, int BM, int BN, int WM, int WN, int NTH, int KA, int EPI, bool EPF, bool EPFB, int SMEM,
+          bool CI = false, int EK = 7, class Acc, int TM, int TN>
+__device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, int z, int zz, int R, int m0, int n0, int tmi, int tid,
+                                              const Acc (&accM)[TM][TN], const Acc (&accV)[TM][TN], float* smem,
+                                              const float* epf_s, const float* epb_h, const float* epb_j) {
+  constexpr int NV = FR * FR / 64;  // outputs per lane and tile
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int wm = wave / (BN / WN);
+  const int wn = wave % (BN / WN);
+  const int hl = lane / FR;
+  const int rl = lane % FR;
+  auto tcol = [&](int j) { return wn * WN + (CI ? rl * TN + j : j * FR + rl); };  // column within the block tile
+  // The epilogue kind is the same
+  // for the whole launch, so each kind gets its own unrolled loop with the per-block
+  // invariants (bias columns, the stride phase and its pixel dividers) hoisted out.
+  const Epi& e = g.epi;
+  if (g.partial) {
+    const int64_t plane = (int64_t)g.R * g.C;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+          const int col = n0 + tcol(j);
+          if (row < R && col < g.C) {
+            const int64_t base = ((int64_t)zz * 2) * plane + (int64_t)row * g.C + col;
+            g.partial[base] = accM[i][j][v];
+            g.partial[base + plane] = accV[i][j][v];
+          }
+        }
+  } else if ((EK & 1) && e.kind == 0 && e.b_sr == 0) {
+    // plain store with an optional per-column bias (Linear, Conv2D forward, bmm)
+    const int64_t zoff = (z / e.zdiv) * e.sz1 + (z % e.zdiv) * e.sz2;
+    const bool st = e.st_ws != nullptr;
+    float* red = smem;  // [BM / WM][3][BN] column sums per wave row (LDS is free here)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int col = n0 + tcol(j);
+      const bool cok = col < g.C;
+      const float bmj = (e.bm && cok) ? e.bm[(int64_t)col * e.b_sc] : 0.f;
+      const float bvj = (e.bv && cok) ? e.bv[(int64_t)col * e.b_sc] : 0.f;
+      const int64_t coff = zoff + (int64_t)col * e.scol;
+      float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        // Multiplier and addend of the lane's outputs are loaded before any store: the
+        // addend may alias the output, so loads issued after a store could not be moved
+        // ahead of it and every element would wait for the previous one's store.
+        // (linear and batched products only: in the conv kernels the extra registers cost
+        // more occupancy than the loads gain)
+        constexpr bool PRE = KA <= LD_STR_K_S;
+        float jv[NV], av0[NV], av1[NV];
+        if (PRE && (e.jm || e.am)) {
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+            const bool ok = row < R && cok;
+            const int64_t off = coff + (int64_t)row * e.srow;
+            jv[v] = (e.jm && ok) ? e.jm[off] : 1.f;
+            av0[v] = (e.am && ok) ? e.am[off] : 0.f;
+            av1[v] = (e.am && ok) ? e.av[off] : 0.f;
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+          if (row < R && cok) {
+            const int64_t off = coff + (int64_t)row * e.srow;
+            float m = accM[i][j][v] * e.sm + bmj, vv = accV[i][j][v] * e.sv + bvj;
+            if (e.jm) {
+              const float jj = PRE ? jv[v] : e.jm[off];
+              m *= jj;
+              vv *= jj * jj;
+            }
+            if (e.am) {
+              m += PRE ? av0[v] : e.am[off];
+              vv += PRE ? av1[v] : e.av[off];
+            }
+            if constexpr (EPI == 4) {
+              float ra, rS, rJ;
+              relu_moments(m, vv, ra, rS, rJ);
+              e.om[off] = ra;
+              e.ov[off] = rS;
+              e.relu_J[off] = rJ;
+              continue;
+            }
+            if (e.om) e.om[off] = m;
+            e.ov[off] = vv;
+            if (st) {
+              float ra, rS, rJ;
+              relu_moments(m, vv, ra, rS, rJ);
+              e.st_J[off] = rJ;
+              s0 += ra;
+              s1 += rS;
+              s2 += ra * ra;
+            }
+          }
+        }
+      }
+      if (st) {
+        // lanes FR apart hold the same column
+#pragma unroll
+        for (int o = FR; o < 64; o <<= 1) {
+          s0 += __shfl_xor(s0, o, 64);
+          s1 += __shfl_xor(s1, o, 64);
+          s2 += __shfl_xor(s2, o, 64);
+        }
+        if (hl == 0) {
+          const int cl = tcol(j);
+          red[(wm * 3 + 0) * BN + cl] = s0;
+          red[(wm * 3 + 1) * BN + cl] = s1;
+          red[(wm * 3 + 2) * BN + cl] = s2;
+        }
+      }
+    }
+    if (st) {
+      __syncthreads();
+      for (int cl = tid; cl < BN; cl += NTH) {
+        const int col = n0 + cl;
+        if (col < g.C) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < BM / WM; ++w) sum += red[(w * 3 + q) * BN + cl];
+            e.st_ws[((int64_t)q * g.C + col) * e.st_nblk + tmi] = sum;
+          }
+        }
+      }
+    }
+  } else if ((EK & 4) && e.kind == 2) {
+    // conv input delta: row q of stride phase z is input pixel (n, hh*s + a, ww*s + b)
+    const Phase ph = make_phase(e.g, z);
+    const int hq = ph.Hq * ph.Wq;
+    const FastDiv dhq = make_fastdiv(hq > 0 ? hq : 1), dwq = make_fastdiv(ph.Wq > 0 ? ph.Wq : 1);
+    // With an addend (the shortcut deltas, possibly the output itself), a lane's addends
+    // of a column are loaded before any of its outputs is stored: a load issued after a
+    // store to a possibly aliasing address would wait for it, element by element.
+    constexpr bool bn = EPI == 1 || EPI == 3;
+    float* red = smem;  // BatchNorm sums: [BM / WM][6][BN] column sums per wave row
+    static_assert(!bn || (BM / WM) * 6 * BN <= SMEM, "BatchNorm sums must fit the LDS tiles");
+    float bsum[TN][6];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int q = 0; q < 6; ++q) bsum[j][q] = 0.f;
+    if constexpr (EPFB) {
+      // m_hat and J are in registers (loaded during the last k-period); EPI 3 loads its
+      // addends 8 at a time, each group before its stores (which may alias them)
+      const int col = n0 + wn * WN + rl;
+      if (col < g.C) {
+        const float rv = e.bn_var[col] + e.bn_eps;
+        const float km = e.bn_g[col] * (1.0f / sqrtf(rv));
+        const float kS = e.bn_g[col] * e.bn_g[col] * (1.0f / rv);
+        float ad0[EPI == 3 ? 8 : 1], ad1[EPI == 3 ? 8 : 1];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + 8 * (v >> 2) + 4 * hl + (v & 3);
+          if constexpr (EPI == 3) {
+            if ((v & 7) == 0) {
+#pragma unroll
+              for (int u = 0; u < 8; ++u) {
+                const int ru = m0 + wm * WM + 8 * ((v + u) >> 2) + 4 * hl + ((v + u) & 3);
+                const int ou = ru * g.C + col;
+                ad0[u] = ru < R ? e.am[ou] : 0.f;
+                ad1[u] = ru < R ? e.av[ou] : 0.f;
+              }
+            }
+          }
+          if (row >= R) continue;
+          const int off = row * g.C + col;
+          float a = accM[0][0][v], b = accV[0][0][v];
+          if constexpr (EPI == 3) {
+            a = a + ad0[v & 7];
+            b = b + ad1[v & 7];
+            e.om[off] = a;
+            e.ov[off] = b;
+          }
+          const float h = epb_h[v], jj = epb_j[v];
+          bsum[0][0] += a * h;
+          bsum[0][1] += b * h * h;
+          bsum[0][2] += a;
+          bsum[0][3] += b;
+          float o0 = a * km, o1 = b * kS;
+          o0 = o0 * jj;
+          o1 = o1 * jj * jj;
+          bsum[0][4] += o0;
+          bsum[0][5] += o1;
+          if constexpr (EPI == 3) {
+            e.bn_om[off] = o0;
+            e.bn_ov[off] = o1;
+          } else {
+            e.om[off] = o0;
+            e.ov[off] = o1;
+          }
+        }
+      }
+    } else
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      int64_t pixc[NV];  // pixel offset * C, or -1 past the phase's rows
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+        const int n = fdiv(row, dhq), rr = row - n * hq;
+        const int hh = fdiv(rr, dwq), ww = rr - hh * ph.Wq;
+        const int64_t pix = ((int64_t)n * e.g.H + (hh * e.g.stride + ph.a)) * e.g.W + (ww * e.g.stride + ph.b);
+        pixc[v] = row < R ? pix * e.g.C : -1;
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int col = n0 + tcol(j);
+        if (col >= g.C) continue;
+        if constexpr (bn) {
+          // the same operations, in the same order, as the separate BatchNorm2D -> ReLU
+          // backward pass (bn_reduce_kernel MODE 4), so the outputs are identical
+          const float rv = e.bn_var[col] + e.bn_eps;
+          const float km = e.bn_g[col] * (1.0f / sqrtf(rv));
+          const float kS = e.bn_g[col] * e.bn_g[col] * (1.0f / rv);
+          // EPI 3 in two halves of 8 outputs (all four operands of 16 at once would cost
+          // occupancy); each half's loads come before its stores, which may alias the addend
+          constexpr int NH = (EPI == 3 && NV == 16) ? 2 : 1, HV = NV / NH;
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh) {
+            float hv[HV], jv[HV], ad0[HV], ad1[HV];
+#pragma unroll
+            for (int u = 0; u < HV; ++u) {
+              const int v = hh * HV + u;
+              hv[u] = pixc[v] >= 0 ? e.bn_mhat[pixc[v] + col] : 0.f;
+              jv[u] = pixc[v] >= 0 ? e.bn_J[pixc[v] + col] : 0.f;
+              if constexpr (EPI == 3) {
+                ad0[u] = pixc[v] >= 0 ? e.am[pixc[v] + col] : 0.f;
+                ad1[u] = pixc[v] >= 0 ? e.av[pixc[v] + col] : 0.f;
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < HV; ++u) {
+              const int v = hh * HV + u;
+              if (pixc[v] < 0) continue;
+              const int64_t off = pixc[v] + col;
+              float a = accM[i][j][v], b = accV[i][j][v];
+              if constexpr (EPI == 3) {
+                a = a + ad0[u];
+                b = b + ad1[u];
+                e.om[off] = a;
+                e.ov[off] = b;
+              }
+              const float h = hv[u], jj = jv[u];
+              bsum[j][0] += a * h;
+              bsum[j][1] += b * h * h;
+              bsum[j][2] += a;
+              bsum[j][3] += b;
+              float o0 = a * km, o1 = b * kS;
+              o0 = o0 * jj;
+              o1 = o1 * jj * jj;
+              bsum[j][4] += o0;
+              bsum[j][5] += o1;
+              if constexpr (EPI == 3) {
+                e.bn_om[off] = o0;
+                e.bn_ov[off] = o1;
+              } else {
+                e.om[off] = o0;
+                e.ov[off] = o1;
+              }
+            }
+          }
+          continue;
+        }
+        float addm[NV], addv[NV];
+        if (e.am) {
+#pragma unroll
+          for (int v = 0; v < NV; ++v) {
+            addm[v] = pixc[v] >= 0 ? e.am[pixc[v] + col] : 0.f;
+            addv[v] = pixc[v] >= 0 ? e.av[pixc[v] + col] : 0.f;
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          if (pixc[v] < 0) continue;
+          const int64_t off = pixc[v] + col;
+          float m = accM[i][j][v], vv = accV[i][j][v];
+          if (e.am) {
+            m = m + addm[v];
+            vv = vv + addv[v];
+          }
+          e.om[off] = m;
+          e.ov[off] = vv;
+        }
+      }
+    }
+    if constexpr (bn) {
+      // lanes FR apart hold the same column; then the tile's wave rows in order
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q)
+#pragma unroll
+          for (int o = FR; o < 64; o <<= 1) bsum[j][q] += __shfl_xor(bsum[j][q], o, 64);
+        if (hl == 0) {
+          const int cl = tcol(j);
+#pragma unroll
+          for (int q = 0; q < 6; ++q) red[(wm * 6 + q) * BN + cl] = bsum[j][q];
+        }
+      }
+      __syncthreads();
+      for (int cl = tid; cl < BN; cl += NTH) {
+        const int col = n0 + cl;
+        if (col < g.C) {
+#pragma unroll
+          for (int q = 0; q < 6; ++q) {
+            float sum = 0.f;
+#pragma unroll
+            for (int w = 0; w < BM / WM; ++w) sum += red[(w * 6 + q) * BN + cl];
+            e.st_ws[((int64_t)q * g.C + col) * e.st_nblk + tmi] = sum;
+          }
+        }
+      }
+    }
+  } else if ((EK & 2) && e.kind == 1) {
+    // parameter deltas (unsplit): the Sw (Sb) factors of a lane's outputs are loaded
+    // before any of them is stored -- the stores may alias them as far as the compiler
+    // knows, so a load issued after a store would wait for it, element by element
+    const bool keep = e.om != nullptr;  // the update without stored deltas: om, dmb null
+    (void)keep;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int col = n0 + tcol(j);
+        if constexpr (EPF) {
+          // the variances were loaded during the last k-period; the means are loaded one
+          // group of 4 ahead of the stores (a load after a store that may alias it would
+          // wait for it)
+          auto widx = [&](int v) -> int64_t {
+            const int row = m0 + wm * WM + 8 * (v >> 2) + 4 * hl + (v & 3);
+            if (!(row < R && col < g.C)) return -2;
+            if (row >= e.wrows) return -1;
+            int wr = row;
+            if (e.perm_C > 0) {
+              const int kidx = fdiv(row, e.dperm);
+              wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
+            }
+            return (int64_t)wr * e.ldw + col;
+          };
+          float pm[4][4];
+          auto load_means = [&](int q) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int64_t w = widx(4 * q + u);
+              pm[q][u] = w >= 0 ? e.upd_mw[w] : (w == -1 ? e.upd_mb[col] : 0.f);
+            }
+          };
+          load_means(0);
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (q < 3) load_means(q + 1);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int64_t w = widx(4 * q + u);
+              if (w == -2) continue;
+              const float sv = epf_s[4 * q + u];
+              const float dm = sv * accM[0][0][4 * q + u], dS = (sv * sv) * accV[0][0][4 * q + u];
+              float pmu = pm[q][u], pS = sv;
+              capped(pmu, pS, dm, dS, e.cap);
+              if (w >= 0) {
+                if (keep) {
+                  e.om[w] = dm;
+                  e.ov[w] = dS;
+                }
+                e.upd_mw[w] = pmu;
+                e.upd_Sw[w] = pS;
+              } else {
+                if (keep) {
+                  e.dmb[col] = dm;
+                  e.dSb[col] = dS;
+                }
+                e.upd_mb[col] = pmu;
+                e.upd_Sb[col] = pS;
+              }
+            }
+          }
+          continue;
+        } else if constexpr (EPI == 2) {
+          // with the capped update in place: per group of 4 outputs, the variances and
+          // means are loaded before the group's stores (16 at once would cost occupancy)
+#pragma unroll
+          for (int q = 0; q < NV / 4; ++q) {
+            float sv4[4], pm4[4];
+            int64_t wi[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int row = m0 + wm * WM + i * FR + 8 * q + 4 * hl + u;
+              sv4[u] = 1.f;
+              pm4[u] = 0.f;
+              wi[u] = -1;
+              if (row < R && col < g.C) {
+                if (row < e.wrows) {
+                  int wr = row;
+                  if (e.perm_C > 0) {
+                    const int kidx = fdiv(row, e.dperm);
+                    wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
+                  }
+                  wi[u] = (int64_t)wr * e.ldw + col;
+                  sv4[u] = e.Sw[wi[u]];
+                  pm4[u] = e.upd_mw[wi[u]];
+                } else {
+                  sv4[u] = e.Sb[col];
+                  pm4[u] = e.upd_mb[col];
+                }
+              }
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int row = m0 + wm * WM + i * FR + 8 * q + 4 * hl + u;
+              if (row < R && col < g.C) {
+                const float sv = sv4[u];
+                const float dm = sv * accM[i][j][4 * q + u], dS = (sv * sv) * accV[i][j][4 * q + u];
+                float pm = pm4[u], pS = sv;
+                capped(pm, pS, dm, dS, e.cap);
+                if (row < e.wrows) {
+                  if (keep) {
+                    e.om[wi[u]] = dm;
+                    e.ov[wi[u]] = dS;
+                  }
+                  e.upd_mw[wi[u]] = pm;
+                  e.upd_Sw[wi[u]] = pS;
+                } else {
+                  if (keep) {
+                    e.dmb[col] = dm;
+                    e.dSb[col] = dS;
+                  }
+                  e.upd_mb[col] = pm;
+                  e.upd_Sb[col] = pS;
+                }
+              }
+            }
+          }
+          continue;
+        }
+        float sf[NV];
+        int64_t widx[NV];
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+          sf[v] = 1.f;
+          widx[v] = -1;
+          if (row < R && col < g.C) {
+            if (row < e.wrows) {
+              int wr = row;
+              if (e.perm_C > 0) {
+                const int kidx = fdiv(row, e.dperm);
+                wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
+              }
+              widx[v] = (int64_t)wr * e.ldw + col;
+              if (e.Sw) sf[v] = e.Sw[widx[v]];
+            } else if (e.Sb) {
+              sf[v] = e.Sb[col];
+            }
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+          if (row < R && col < g.C) {
+            const float sv = sf[v];
+            if (row < e.wrows) {
+              e.om[widx[v]] = sv * accM[i][j][v];
+              e.ov[widx[v]] = (sv * sv) * accV[i][j][v];
+            } else {
+              e.dmb[col] = sv * accM[i][j][v];
+              e.dSb[col] = (sv * sv) * accV[i][j][v];
+            }
+          }
+        }
+      }
+  } else if constexpr (EK == 7) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) {
+          const int row = m0 + wm * WM + i * FR + 8 * (v >> 2) + 4 * hl + (v & 3);
+          const int col = n0 + tcol(j);
+          if (row < R && col < g.C) epi_apply(e, z, row, col, accM[i][j][v], accV[i][j][v]);
+        }
+  }
+}
+
 // EPI 1: the kind-2 epilogue with the BatchNorm2D -> ReLU backward folded in; EPI 2: the
 // kind-1 epilogue with the capped parameter update applied in place; EPI 3: EPI 1 applied
 // to product + addend, storing both; EPI 4: the kind-0 plain store of ReLU(product)'s
@@ -912,57 +1721,10 @@ __global__ void __launch_bounds__(CFG::NTH, ((EPI == 1 || EPI == 3) && CFG::NTH 
   const int hl = lane >> 5;
   const int rl = lane & 31;
 
-  // Split-K launches with at least 8 split groups: every tile of one split group (the
-  // tiles that read the same stretch of the reduction) goes to one XCD. Workgroups are
-  // dealt round-robin over the 8 XCDs in linear-id order, so the linear id L is read as
-  // (XCD x = L mod 8, k-th block of that XCD) and group 8*(k / nt) + x, tile k mod nt
-  // are assigned; groups past the last multiple of 8 keep the plain order. Without this,
-  // the tiles of a group land on different XCDs and each XCD's L2 fetches the shared
-  // operand panels again (the parameter-delta GEMMs' 9 tap tiles share one pixel range).
-  int zq, split, bid;
-  bool xcd_tiles = true;
-  if (!g.phased && g.splits > 1 && gridDim.y >= 8 && (uint64_t)gridDim.x * gridDim.y < (1ull << 31)) {
-    const int nt0 = g.tiles_m * g.tiles_n;
-    const int L = blockIdx.x + blockIdx.y * gridDim.x;
-    const int g8 = (int)(gridDim.y & ~7u);
-    int grp, tile;
-    if (L < g8 * nt0) {
-      const int k = L >> 3, q = k / nt0;
-      grp = q * 8 + (L & 7);
-      tile = k - q * nt0;
-    } else {
-      const int L2 = L - g8 * nt0, q = L2 / nt0;
-      grp = g8 + q;
-      tile = L2 - q * nt0;
-    }
-    zq = grp / g.splits;
-    split = grp - zq * g.splits;
-    bid = tile;
-    xcd_tiles = false;
-  } else {
-    zq = blockIdx.y / g.splits;
-    split = blockIdx.y - zq * g.splits;
-    bid = blockIdx.x;
-  }
-  const int z = g.phased ? (int)g.phase_order[zq] : zq;
-  const int zz = z * g.splits + split;  // partial-sum slot
-  const int R = rows_of(g, z);
-  const int Kred = kred_of(g, z);
-  const int tiles_m = g.phased ? (R + BM - 1) / BM : g.tiles_m;
-
-  // XCD-aware tile order: workgroups are dealt round-robin over the 8 XCDs, so map
-  // consecutive block ids of one XCD onto consecutive tiles (shared operand panels stay
-  // in that XCD's L2).
-  const int nt = tiles_m * g.tiles_n;
-  if (bid >= nt) return;  // phased launches size the grid for the largest phase
-  const int per = nt >> 3;
-  const int t = (xcd_tiles && bid < (per << 3)) ? ((bid & 7) * per + (bid >> 3)) : bid;
-  const int tmi = t / g.tiles_n;
-  const int tni = t - tmi * g.tiles_n;
-  const int m0 = tmi * BM;
-  const int n0 = tni * BN;
-  const int kbeg = split * g.k_chunk;
-  const int kend = min(Kred, kbeg + g.k_chunk);
+  BlockPos bp;
+  if (!block_pos<BM, BN>(g, bp)) return;
+  const int z = bp.z, R = bp.R, tmi = bp.tmi, m0 = bp.m0, n0 = bp.n0, kbeg = bp.kbeg, kend = bp.kend;
+  const int zz = z * g.splits + bp.split;  // partial-sum slot
 
   LA la;
   LB lb;
@@ -1226,478 +1988,8 @@ __global__ void __launch_bounds__(CFG::NTH, ((EPI == 1 || EPI == 3) && CFG::NTH 
     }
   }
 
-  // Epilogue: split-K partial sums, or the layer's epilogue. The epilogue kind is the same
-  // for the whole launch, so each kind gets its own unrolled loop with the per-block
-  // invariants (bias columns, the stride phase and its pixel dividers) hoisted out.
-  const Epi& e = g.epi;
-  if (g.partial) {
-    const int64_t plane = (int64_t)g.R * g.C;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-          const int col = n0 + wn * WN + j * 32 + rl;
-          if (row < R && col < g.C) {
-            const int64_t base = ((int64_t)zz * 2) * plane + (int64_t)row * g.C + col;
-            g.partial[base] = accM[i][j][v];
-            g.partial[base + plane] = accV[i][j][v];
-          }
-        }
-  } else if (e.kind == 0 && e.b_sr == 0) {
-    // plain store with an optional per-column bias (Linear, Conv2D forward, bmm)
-    const int64_t zoff = (z / e.zdiv) * e.sz1 + (z % e.zdiv) * e.sz2;
-    const bool st = e.st_ws != nullptr;
-    float* red = smem;  // [BM / WM][3][BN] column sums per wave row (LDS is free here)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = n0 + wn * WN + j * 32 + rl;
-      const bool cok = col < g.C;
-      const float bmj = (e.bm && cok) ? e.bm[(int64_t)col * e.b_sc] : 0.f;
-      const float bvj = (e.bv && cok) ? e.bv[(int64_t)col * e.b_sc] : 0.f;
-      const int64_t coff = zoff + (int64_t)col * e.scol;
-      float s0 = 0.f, s1 = 0.f, s2 = 0.f;
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        // Multiplier and addend of the lane's 16 outputs are loaded before any store: the
-        // addend may alias the output, so loads issued after a store could not be moved
-        // ahead of it and every element would wait for the previous one's store.
-        // (linear and batched products only: in the conv kernels the extra registers cost
-        // more occupancy than the loads gain)
-        constexpr bool PRE = KA <= LD_STR_K_S;
-        float jv[16], av0[16], av1[16];
-        if (PRE && (e.jm || e.am)) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-            const bool ok = row < R && cok;
-            const int64_t off = coff + (int64_t)row * e.srow;
-            jv[v] = (e.jm && ok) ? e.jm[off] : 1.f;
-            av0[v] = (e.am && ok) ? e.am[off] : 0.f;
-            av1[v] = (e.am && ok) ? e.av[off] : 0.f;
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-          if (row < R && cok) {
-            const int64_t off = coff + (int64_t)row * e.srow;
-            float m = accM[i][j][v] * e.sm + bmj, vv = accV[i][j][v] * e.sv + bvj;
-            if (e.jm) {
-              const float jj = PRE ? jv[v] : e.jm[off];
-              m *= jj;
-              vv *= jj * jj;
-            }
-            if (e.am) {
-              m += PRE ? av0[v] : e.am[off];
-              vv += PRE ? av1[v] : e.av[off];
-            }
-            if constexpr (EPI == 4) {
-              float ra, rS, rJ;
-              relu_moments(m, vv, ra, rS, rJ);
-              e.om[off] = ra;
-              e.ov[off] = rS;
-              e.relu_J[off] = rJ;
-              continue;
-            }
-            if (e.om) e.om[off] = m;
-            e.ov[off] = vv;
-            if (st) {
-              float ra, rS, rJ;
-              relu_moments(m, vv, ra, rS, rJ);
-              e.st_J[off] = rJ;
-              s0 += ra;
-              s1 += rS;
-              s2 += ra * ra;
-            }
-          }
-        }
-      }
-      if (st) {
-        // lanes l and l + 32 hold the same column
-        s0 += __shfl_xor(s0, 32, 64);
-        s1 += __shfl_xor(s1, 32, 64);
-        s2 += __shfl_xor(s2, 32, 64);
-        if (hl == 0) {
-          const int cl = wn * WN + j * 32 + rl;
-          red[(wm * 3 + 0) * BN + cl] = s0;
-          red[(wm * 3 + 1) * BN + cl] = s1;
-          red[(wm * 3 + 2) * BN + cl] = s2;
-        }
-      }
-    }
-    if (st) {
-      __syncthreads();
-      for (int cl = tid; cl < BN; cl += NTH) {
-        const int col = n0 + cl;
-        if (col < g.C) {
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            float sum = 0.f;
-#pragma unroll
-            for (int w = 0; w < BM / WM; ++w) sum += red[(w * 3 + q) * BN + cl];
-            e.st_ws[((int64_t)q * g.C + col) * e.st_nblk + tmi] = sum;
-          }
-        }
-      }
-    }
-  } else if (e.kind == 2) {
-    // conv input delta: row q of stride phase z is input pixel (n, hh*s + a, ww*s + b)
-    const Phase ph = make_phase(e.g, z);
-    const int hq = ph.Hq * ph.Wq;
-    const FastDiv dhq = make_fastdiv(hq > 0 ? hq : 1), dwq = make_fastdiv(ph.Wq > 0 ? ph.Wq : 1);
-    // With an addend (the shortcut deltas, possibly the output itself), a lane's 16 addends
-    // of a column are loaded before any of its outputs is stored: a load issued after a
-    // store to a possibly aliasing address would wait for it, element by element.
-    constexpr bool bn = EPI == 1 || EPI == 3;
-    float* red = smem;  // BatchNorm sums: [BM / WM][6][BN] column sums per wave row
-    static_assert((BM / WM) * 6 * BN <= 2 * (SA + SB), "BatchNorm sums must fit the LDS tiles");
-    float bsum[TN][6];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int q = 0; q < 6; ++q) bsum[j][q] = 0.f;
-    if constexpr (EPFB) {
-      // m_hat and J are in registers (loaded during the last k-period); EPI 3 loads its
-      // addends 8 at a time, each group before its stores (which may alias them)
-      const int col = n0 + wn * WN + rl;
-      if (col < g.C) {
-        const float rv = e.bn_var[col] + e.bn_eps;
-        const float km = e.bn_g[col] * (1.0f / sqrtf(rv));
-        const float kS = e.bn_g[col] * e.bn_g[col] * (1.0f / rv);
-        float ad0[EPI == 3 ? 8 : 1], ad1[EPI == 3 ? 8 : 1];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + 8 * (v >> 2) + 4 * hl + (v & 3);
-          if constexpr (EPI == 3) {
-            if ((v & 7) == 0) {
-#pragma unroll
-              for (int u = 0; u < 8; ++u) {
-                const int ru = m0 + wm * WM + 8 * ((v + u) >> 2) + 4 * hl + ((v + u) & 3);
-                const int ou = ru * g.C + col;
-                ad0[u] = ru < R ? e.am[ou] : 0.f;
-                ad1[u] = ru < R ? e.av[ou] : 0.f;
-              }
-            }
-          }
-          if (row >= R) continue;
-          const int off = row * g.C + col;
-          float a = accM[0][0][v], b = accV[0][0][v];
-          if constexpr (EPI == 3) {
-            a = a + ad0[v & 7];
-            b = b + ad1[v & 7];
-            e.om[off] = a;
-            e.ov[off] = b;
-          }
-          const float h = epb_h[v], jj = epb_j[v];
-          bsum[0][0] += a * h;
-          bsum[0][1] += b * h * h;
-          bsum[0][2] += a;
-          bsum[0][3] += b;
-          float o0 = a * km, o1 = b * kS;
-          o0 = o0 * jj;
-          o1 = o1 * jj * jj;
-          bsum[0][4] += o0;
-          bsum[0][5] += o1;
-          if constexpr (EPI == 3) {
-            e.bn_om[off] = o0;
-            e.bn_ov[off] = o1;
-          } else {
-            e.om[off] = o0;
-            e.ov[off] = o1;
-          }
-        }
-      }
-    } else
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      int64_t pixc[16];  // pixel offset * C, or -1 past the phase's rows
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-        const int n = fdiv(row, dhq), rr = row - n * hq;
-        const int hh = fdiv(rr, dwq), ww = rr - hh * ph.Wq;
-        const int64_t pix = ((int64_t)n * e.g.H + (hh * e.g.stride + ph.a)) * e.g.W + (ww * e.g.stride + ph.b);
-        pixc[v] = row < R ? pix * e.g.C : -1;
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wn * WN + j * 32 + rl;
-        if (col >= g.C) continue;
-        if constexpr (bn) {
-          // the same operations, in the same order, as the separate BatchNorm2D -> ReLU
-          // backward pass (bn_reduce_kernel MODE 4), so the outputs are identical
-          const float rv = e.bn_var[col] + e.bn_eps;
-          const float km = e.bn_g[col] * (1.0f / sqrtf(rv));
-          const float kS = e.bn_g[col] * e.bn_g[col] * (1.0f / rv);
-          // EPI 3 in two halves of 8 outputs (all four operands of 16 at once would cost
-          // occupancy); each half's loads come before its stores, which may alias the addend
-          constexpr int NH = EPI == 3 ? 2 : 1, HV = 16 / NH;
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh) {
-            float hv[HV], jv[HV], ad0[HV], ad1[HV];
-#pragma unroll
-            for (int u = 0; u < HV; ++u) {
-              const int v = hh * HV + u;
-              hv[u] = pixc[v] >= 0 ? e.bn_mhat[pixc[v] + col] : 0.f;
-              jv[u] = pixc[v] >= 0 ? e.bn_J[pixc[v] + col] : 0.f;
-              if constexpr (EPI == 3) {
-                ad0[u] = pixc[v] >= 0 ? e.am[pixc[v] + col] : 0.f;
-                ad1[u] = pixc[v] >= 0 ? e.av[pixc[v] + col] : 0.f;
-              }
-            }
-#pragma unroll
-            for (int u = 0; u < HV; ++u) {
-              const int v = hh * HV + u;
-              if (pixc[v] < 0) continue;
-              const int64_t off = pixc[v] + col;
-              float a = accM[i][j][v], b = accV[i][j][v];
-              if constexpr (EPI == 3) {
-                a = a + ad0[u];
-                b = b + ad1[u];
-                e.om[off] = a;
-                e.ov[off] = b;
-              }
-              const float h = hv[u], jj = jv[u];
-              bsum[j][0] += a * h;
-              bsum[j][1] += b * h * h;
-              bsum[j][2] += a;
-              bsum[j][3] += b;
-              float o0 = a * km, o1 = b * kS;
-              o0 = o0 * jj;
-              o1 = o1 * jj * jj;
-              bsum[j][4] += o0;
-              bsum[j][5] += o1;
-              if constexpr (EPI == 3) {
-                e.bn_om[off] = o0;
-                e.bn_ov[off] = o1;
-              } else {
-                e.om[off] = o0;
-                e.ov[off] = o1;
-              }
-            }
-          }
-          continue;
-        }
-        float addm[16], addv[16];
-        if (e.am) {
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            addm[v] = pixc[v] >= 0 ? e.am[pixc[v] + col] : 0.f;
-            addv[v] = pixc[v] >= 0 ? e.av[pixc[v] + col] : 0.f;
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          if (pixc[v] < 0) continue;
-          const int64_t off = pixc[v] + col;
-          float m = accM[i][j][v], vv = accV[i][j][v];
-          if (e.am) {
-            m = m + addm[v];
-            vv = vv + addv[v];
-          }
-          e.om[off] = m;
-          e.ov[off] = vv;
-        }
-      }
-    }
-    if constexpr (bn) {
-      // lanes l and l + 32 hold the same column; then the tile's wave rows in order
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-#pragma unroll
-        for (int q = 0; q < 6; ++q) bsum[j][q] += __shfl_xor(bsum[j][q], 32, 64);
-        if (hl == 0) {
-          const int cl = wn * WN + j * 32 + rl;
-#pragma unroll
-          for (int q = 0; q < 6; ++q) red[(wm * 6 + q) * BN + cl] = bsum[j][q];
-        }
-      }
-      __syncthreads();
-      for (int cl = tid; cl < BN; cl += NTH) {
-        const int col = n0 + cl;
-        if (col < g.C) {
-#pragma unroll
-          for (int q = 0; q < 6; ++q) {
-            float sum = 0.f;
-#pragma unroll
-            for (int w = 0; w < BM / WM; ++w) sum += red[(w * 6 + q) * BN + cl];
-            e.st_ws[((int64_t)q * g.C + col) * e.st_nblk + tmi] = sum;
-          }
-        }
-      }
-    }
-  } else if (e.kind == 1) {
-    // parameter deltas (unsplit): the Sw (Sb) factors of a lane's 16 outputs are loaded
-    // before any of them is stored -- the stores may alias them as far as the compiler
-    // knows, so a load issued after a store would wait for it, element by element
-    const bool keep = e.om != nullptr;  // the update without stored deltas: om, dmb null
-    (void)keep;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int col = n0 + wn * WN + j * 32 + rl;
-        if constexpr (EPF) {
-          // the variances were loaded during the last k-period; the means are loaded one
-          // group of 4 ahead of the stores (a load after a store that may alias it would
-          // wait for it)
-          auto widx = [&](int v) -> int64_t {
-            const int row = m0 + wm * WM + 8 * (v >> 2) + 4 * hl + (v & 3);
-            if (!(row < R && col < g.C)) return -2;
-            if (row >= e.wrows) return -1;
-            int wr = row;
-            if (e.perm_C > 0) {
-              const int kidx = fdiv(row, e.dperm);
-              wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
-            }
-            return (int64_t)wr * e.ldw + col;
-          };
-          float pm[4][4];
-          auto load_means = [&](int q) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int64_t w = widx(4 * q + u);
-              pm[q][u] = w >= 0 ? e.upd_mw[w] : (w == -1 ? e.upd_mb[col] : 0.f);
-            }
-          };
-          load_means(0);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            if (q < 3) load_means(q + 1);
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int64_t w = widx(4 * q + u);
-              if (w == -2) continue;
-              const float sv = epf_s[4 * q + u];
-              const float dm = sv * accM[0][0][4 * q + u], dS = (sv * sv) * accV[0][0][4 * q + u];
-              float pmu = pm[q][u], pS = sv;
-              capped(pmu, pS, dm, dS, e.cap);
-              if (w >= 0) {
-                if (keep) {
-                  e.om[w] = dm;
-                  e.ov[w] = dS;
-                }
-                e.upd_mw[w] = pmu;
-                e.upd_Sw[w] = pS;
-              } else {
-                if (keep) {
-                  e.dmb[col] = dm;
-                  e.dSb[col] = dS;
-                }
-                e.upd_mb[col] = pmu;
-                e.upd_Sb[col] = pS;
-              }
-            }
-          }
-          continue;
-        } else if constexpr (EPI == 2) {
-          // with the capped update in place: per group of 4 outputs, the variances and
-          // means are loaded before the group's stores (16 at once would cost occupancy)
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            float sv4[4], pm4[4];
-            int64_t wi[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int row = m0 + wm * WM + i * 32 + 8 * q + 4 * hl + u;
-              sv4[u] = 1.f;
-              pm4[u] = 0.f;
-              wi[u] = -1;
-              if (row < R && col < g.C) {
-                if (row < e.wrows) {
-                  int wr = row;
-                  if (e.perm_C > 0) {
-                    const int kidx = fdiv(row, e.dperm);
-                    wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
-                  }
-                  wi[u] = (int64_t)wr * e.ldw + col;
-                  sv4[u] = e.Sw[wi[u]];
-                  pm4[u] = e.upd_mw[wi[u]];
-                } else {
-                  sv4[u] = e.Sb[col];
-                  pm4[u] = e.upd_mb[col];
-                }
-              }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int row = m0 + wm * WM + i * 32 + 8 * q + 4 * hl + u;
-              if (row < R && col < g.C) {
-                const float sv = sv4[u];
-                const float dm = sv * accM[i][j][4 * q + u], dS = (sv * sv) * accV[i][j][4 * q + u];
-                float pm = pm4[u], pS = sv;
-                capped(pm, pS, dm, dS, e.cap);
-                if (row < e.wrows) {
-                  if (keep) {
-                    e.om[wi[u]] = dm;
-                    e.ov[wi[u]] = dS;
-                  }
-                  e.upd_mw[wi[u]] = pm;
-                  e.upd_Sw[wi[u]] = pS;
-                } else {
-                  if (keep) {
-                    e.dmb[col] = dm;
-                    e.dSb[col] = dS;
-                  }
-                  e.upd_mb[col] = pm;
-                  e.upd_Sb[col] = pS;
-                }
-              }
-            }
-          }
-          continue;
-        }
-        float sf[16];
-        int64_t widx[16];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-          sf[v] = 1.f;
-          widx[v] = -1;
-          if (row < R && col < g.C) {
-            if (row < e.wrows) {
-              int wr = row;
-              if (e.perm_C > 0) {
-                const int kidx = fdiv(row, e.dperm);
-                wr = (row - kidx * e.perm_C) * e.perm_kk2 + kidx;
-              }
-              widx[v] = (int64_t)wr * e.ldw + col;
-              if (e.Sw) sf[v] = e.Sw[widx[v]];
-            } else if (e.Sb) {
-              sf[v] = e.Sb[col];
-            }
-          }
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-          if (row < R && col < g.C) {
-            const float sv = sf[v];
-            if (row < e.wrows) {
-              e.om[widx[v]] = sv * accM[i][j][v];
-              e.ov[widx[v]] = (sv * sv) * accV[i][j][v];
-            } else {
-              e.dmb[col] = sv * accM[i][j][v];
-              e.dSb[col] = (sv * sv) * accV[i][j][v];
-            }
-          }
-        }
-      }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const int row = m0 + wm * WM + i * 32 + 8 * (v >> 2) + 4 * hl + (v & 3);
-          const int col = n0 + wn * WN + j * 32 + rl;
-          if (row < R && col < g.C) epi_apply(e, z, row, col, accM[i][j][v], accV[i][j][v]);
-        }
-  }
+  gemm_epilogue<32, BM, BN, WM, WN, NTH, KA, EPI, EPF, EPFB, 2 * (SA + SB)>(g, z, zz, R, m0, n0, tmi, tid, accM, accV, smem,
+                                                                          epf_s, epb_h, epb_j);
 }
 
 // Deterministic split-K reduction followed by the epilogue. A block owns 64*V consecutive
@@ -1811,18 +2103,126 @@ using C64x64 = Cfg<64, 64, 32, 32>;      // 4 waves
 using C32x32 = Cfg<32, 32, 32, 32>;      // 1 wave
 using C128x32 = Cfg<128, 32, 32, 32>;    // 4 waves stacked along M (products with 32 columns)
 
+using X256x128 = XCfg<8, 32, 128, 2, 2, 2, 2>;
+using X256x64 = XCfg<8, 32, 64, 2, 2, 2, 2>;
+using X128x128 = XCfg<8, 16, 128, 2, 2, 1, 4>;
+using X128x64 = XCfg<4, 32, 64, 1, 2, 1, 3>;
+using X64x64 = XCfg<4, 16, 64, 1, 4, 1, 4>;
+using X128x32 = XCfg<4, 32, 32, 2, 3, 2, 3>;
+using X64x32 = XCfg<4, 16, 32, 2, 4, 2, 4>;
+using X32x32 = XCfg<2, 16, 32, 1, 4, 1, 4>;
+
+// Tile configs: 0-5 the fp32 kernel's, from 6 on the split kernel's, whose BM is the direct
+// operand's side (the tile's columns when that is B).
 struct CfgDesc {
-  int BM, BN;
+  int BM, BN, BK;
 };
-static const CfgDesc kCfg[] = {{128, 128}, {128, 64}, {64, 128}, {64, 64}, {32, 32}, {128, 32}};
-static const int kNumCfg = 6;
+static const CfgDesc kCfg[] = {{128, 128, 16}, {128, 64, 16}, {64, 128, 16}, {64, 64, 16}, {32, 32, 16},
+                               {128, 32, 16},  {256, 128, 32}, {256, 64, 32}, {128, 128, 32}, {128, 64, 32},
+                               {64, 64, 32},   {128, 32, 32},  {64, 32, 32},  {32, 32, 32}};
+static const int kNumCfg32 = 6, kNumCfg = 14;
+// which operand the split kernel reads directly (0: the product has no split kernel)
+// (XD_SCALAR, with XD_A: that operand's conv patches are read element by element)
+enum { XD_NONE = 0, XD_A = 1, XD_B = 2, XD_SCALAR = 4 };
+static inline int cfg_bm(int c, int xd) { return c >= kNumCfg32 && xd == XD_B ? kCfg[c].BN : kCfg[c].BM; }
+static inline int cfg_bn(int c, int xd) { return c >= kNumCfg32 && xd == XD_B ? kCfg[c].BM : kCfg[c].BN; }
 
 struct Plan {
   int cfg;
   int splits;
   int k_chunk;
   int tiles_m, tiles_n;
+  int xd;  // the call's direct operand (XD_*)
 };
+
+// Whether a product with a split kernel runs it (else the fp32 kernel). The split kernel is
+// the faster one wherever the matrix cores or the loads' volume bound the launch, 1.2 to 1.8
+// times at 2^28 multiply-adds and more, and no slower on small products with a short
+// reduction (their k tiles are twice as long, so there are half as many). Not on
+//   * few multiply-adds over a long reduction, which both kernels cut into many splits whose
+//     chains of loads and barriers are the time: the fp32 kernel's 16-wide k tiles give the
+//     shorter chain (256 x 784 x 256 forward 15.5 against 16.5 us, its parameter deltas 13.8
+//     against 14.7; 128 x 1024 x 256 14.1 against 14.7);
+//   * element-wise patches under one k tile (a 3-channel 3 x 3 input at 131072 pixels: 28.9
+//     against 33.3 us);
+//   * sides under 4, which its float4 loads of any alignment do not cover.
+static inline bool use_split(int64_t R, int64_t C, int64_t Kred, int64_t batch, int xd, bool narrow) {
+  if (xd == XD_NONE || narrow) return false;
+  if (Kred >= 256 && (double)R * C * Kred * batch < (double)(1 << 26)) return false;
+  return !((xd & XD_SCALAR) && Kred < 32);
+}
+
+// The split kernel's plan, from the same kind of model as the fp32 kernel's below: blocks run
+// in rounds of 256 CUs x resident blocks; r blocks on a CU take the larger (as a 4-norm, for
+// the transition) of r times a block's work at the sustained rate and of one block's chain
+// over its k tiles. Rates (relative to the fp32 MFMA peak), chain times per 32-wide k tile,
+// the time per output element, per element-wise patch element and per partial-sum byte were
+// fitted to a sweep of every tile shape and 18 split counts over 158 Linear and Conv2D
+// products on MI355X; the plan picked is 3.1% slower than the best measured one on average,
+// 22% at worst.
+static inline Plan choose_split_plan(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, int64_t max_sp,
+                                     const int64_t* phase_k, int xd) {
+  // [split tile config][product: forward, shared B, shared A]
+  static const int kBpc[8][3] = {{1, 1, 1}, {1, 1, 1}, {1, 2, 2}, {2, 3, 3}, {4, 4, 4}, {3, 3, 3}, {4, 4, 4}, {8, 8, 8}};
+  static const double kEff[8][3] = {{1.46, 1.80, 2.03},
+                                    {1.53, 1.33, 1.64},
+                                    {1.64, 1.59, 1.52},
+                                    {1.40, 1.35, 1.33},
+                                    {1.24, 1.14, 1.14},
+                                    {1.04, 0.91, 0.95},
+                                    {0.77, 0.80, 0.75},
+                                    {0.68, 0.61, 0.57}};
+  static const double kChain[8][3] = {{1.66e-6, 4.21e-6, 4.57e-6},
+                                    {3.43e-6, 2.35e-6, 2.81e-6},
+                                    {3.63e-6, 2.88e-6, 3.75e-6},
+                                    {3.15e-6, 2.59e-6, 2.68e-6},
+                                    {2.26e-6, 1.57e-6, 1.75e-6},
+                                    {2.40e-6, 1.51e-6, 1.86e-6},
+                                    {1.71e-6, 1.04e-6, 1.44e-6},
+                                    {1.58e-6, 0.91e-6, 1.14e-6}};
+  static const int kSplits[] = {1,  2,  3,  4,  5,  6,   8,   10,  12,  16,  20,  24,  32,
+                                40, 48, 64, 80, 96, 128, 160, 192, 256, 320, 384, 512};
+  const double peak_cu = 157.3e12 / 256.0;
+  const double kFixed = 0.24e-6, kOut = 4.26e-10, kDecode = 3.52e-10, kSplitSecPerByte = 1.25e-13, kSplitLaunch = 2.0e-6;
+  const int products = prod == PROD_FWD ? 3 : 2;
+  const int side = xd & (XD_A | XD_B);
+  Plan best{};
+  double best_t = DBL_MAX;
+  for (int x = 0; x < kNumCfg - kNumCfg32; ++x) {
+    const int ci = kNumCfg32 + x, BM = cfg_bm(ci, side), BN = cfg_bn(ci, side), bpc = kBpc[x][prod];
+    const int64_t tm = cdiv(R, BM), tn = cdiv(C, BN);
+    int64_t prev = -1;
+    for (int si = 0; si < (int)(sizeof(kSplits) / sizeof(kSplits[0])) && kSplits[si] <= max_sp; ++si) {
+      const int64_t kc = cdiv(cdiv(Kred, kSplits[si]), 32) * 32, actual = cdiv(Kred, kc);
+      if (actual == prev) continue;
+      prev = actual;
+      int64_t blocks = tm * tn * batch * actual;
+      if (phase_k) {
+        // phases with a shorter reduction do that fraction of a kc block's work
+        double eq = 0.0;
+        for (int64_t z = 0; z < batch; ++z) eq += (double)(tm * tn) * (phase_k[z] > 0 ? (double)phase_k[z] / kc : 0.1);
+        blocks = (int64_t)ceil(eq);
+      }
+      double block_s = (2.0 * BM * BN * kc * products) / (peak_cu * kEff[x][prod]) + BM * BN * kOut;
+      if (xd & XD_SCALAR) block_s += kCfg[ci].BM * (double)kc * kDecode;
+      const double chain = kFixed + (double)(kc / 32) * kChain[x][prod];
+      auto round_s = [&](double r) {
+        const double a = r * block_s * r * block_s, b = chain * chain;
+        return sqrt(sqrt(a * a + b * b));
+      };
+      const int64_t full = blocks / (256 * bpc), rem = blocks - full * 256 * bpc;
+      double t = (double)full * round_s(bpc) + (rem > 0 ? round_s((double)cdiv(rem, 256)) : 0.0);
+      // (an unsplit conv input delta also carries the folded BatchNorm2D backward, which a
+      // split one leaves to two more passes)
+      if (actual > 1) t += (double)actual * 16.0 * R * C * batch * kSplitSecPerByte + (phase_k ? 3.0 : 1.0) * kSplitLaunch;
+      if (t < best_t * 0.999) {
+        best_t = t;
+        best = Plan{ci, (int)actual, (int)kc, (int)tm, (int)tn, side};
+      }
+    }
+  }
+  return best;
+}
 
 // Pick the tile shape and split-K factor minimising a time model of the launch:
 //   * blocks run in rounds of 256 CUs x (resident blocks per CU); a partial last round
@@ -1846,7 +2246,7 @@ struct Plan {
 // phase_k (optional, batch entries): per-GEMM reduction lengths when they differ (stride
 // phases of the conv input delta); splits past a GEMM's own length launch no work.
 static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, bool allow_split,
-                                        int64_t max_splits, const int64_t* phase_k) {
+                                        int64_t max_splits, const int64_t* phase_k, int xd, bool narrow) {
   // [tile config][product: forward, shared B, shared A]
   static const int kBpc[6][3] = {{1, 1, 1}, {2, 3, 3}, {2, 3, 2}, {4, 4, 4}, {8, 10, 10}, {3, 4, 4}};
   static const double kEff[6][3] = {{0.624, 0.353, 0.483}, {0.595, 0.632, 0.608}, {0.465, 0.519, 0.492},
@@ -1868,11 +2268,12 @@ static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int6
   const double kChainFixed = 3.5e-6, kSplitLaunchSmall = 3.0e-6;
   const bool small = !phase_k && cdiv(R, 64) * cdiv(C, 64) * batch < 128;
   const int products = prod == PROD_FWD ? 3 : 2;
-  Plan best{3, 1, (int)Kred, 1, 1};
+  Plan best{3, 1, (int)Kred, 1, 1, XD_NONE};
   double best_t = DBL_MAX;
   const double peak_cu = 157.3e12 / 256.0;
   const int64_t max_sp = allow_split ? (max_splits < 512 ? max_splits : 512) : 1;
-  for (int ci = 0; ci < kNumCfg; ++ci) {
+  if (use_split(R, C, Kred, batch, xd, narrow)) return choose_split_plan(R, C, Kred, batch, prod, max_sp, phase_k, xd);
+  for (int ci = 0; ci < kNumCfg32; ++ci) {
     const int BM = kCfg[ci].BM, BN = kCfg[ci].BN;
     const int64_t tm = cdiv(R, BM), tn = cdiv(C, BN);
     const int bpc = kBpc[ci][prod];
@@ -1909,7 +2310,7 @@ static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int6
         t += (double)actual * 16.0 * R * C * batch * kSplitSecPerByte + (small ? kSplitLaunchSmall : kSplitLaunch);
       if (t < best_t * 0.999) {
         best_t = t;
-        best = Plan{ci, (int)actual, (int)kc, (int)tm, (int)tn};
+        best = Plan{ci, (int)actual, (int)kc, (int)tm, (int)tn, XD_NONE};
       }
     }
   }
@@ -1919,10 +2320,10 @@ static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int6
 // Plans are pure functions of the problem shape; memoise them per host thread (the
 // search above costs a few microseconds and the same shapes recur every step).
 static inline Plan choose_plan(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, bool allow_split,
-                               int64_t max_splits, const int64_t* phase_k = nullptr) {
+                               int64_t max_splits, const int64_t* phase_k = nullptr, int xd = XD_NONE, bool narrow = false) {
   struct Key {
     int64_t R, C, K, batch, max_splits, salt;
-    int prod, allow;
+    int prod, allow, xd;
   };
   int64_t salt = 0;
   if (phase_k)
@@ -1933,14 +2334,14 @@ static inline Plan choose_plan(int64_t R, int64_t C, int64_t Kred, int64_t batch
   };
   static thread_local Entry cache[64];
   static thread_local int used = 0, next = 0;
-  const Key key{R, C, Kred, batch, max_splits, salt, prod, allow_split ? 1 : 0};
+  const Key key{R, C, Kred, batch, max_splits, salt, prod, allow_split ? 1 : 0, xd + (narrow ? 8 : 0)};
   for (int i = 0; i < used; ++i) {
     const Key& k = cache[i].k;
     if (k.R == R && k.C == C && k.K == Kred && k.batch == batch && k.max_splits == max_splits && k.salt == salt &&
-        k.prod == prod && k.allow == key.allow)
+        k.prod == prod && k.allow == key.allow && k.xd == key.xd)
       return cache[i].p;
   }
-  const Plan p = choose_plan_uncached(R, C, Kred, batch, prod, allow_split, max_splits, phase_k);
+  const Plan p = choose_plan_uncached(R, C, Kred, batch, prod, allow_split, max_splits, phase_k, xd, narrow);
   cache[next] = Entry{key, p};
   next = (next + 1) % 64;
   if (used < 64) ++used;
@@ -1977,14 +2378,14 @@ static inline int64_t plan_ws_bytes(const Plan& p, int64_t R, int64_t C, int64_t
   X(PROD_SHARED_A, LD_CWG_A4, LD_STR_MN4) X(PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN4)       \
   X(PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN_S)                                              \
   X(PROD_SHARED_A, LD_STR_MN4, LD_STR_MN4) X(PROD_SHARED_A, LD_STR_MN_S, LD_STR_MN_S)    \
-  X(PROD_SHARED_A, LD_STR_K4, LD_STR_K4) X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4)         \
+  X(PROD_SHARED_A, LD_STR_K_S, LD_STR_MN_S) X(PROD_SHARED_A, LD_STR_K4, LD_STR_K4) X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4)         \
   X(PROD_SHARED_A, LD_STR_MN4, LD_STR_K4)
 
 // The input-delta loader pairs that also get the folded BatchNorm2D epilogues (EPI 1 and
 // 3), in the tile configs with one 32 x 32 tile per wave (64 x 64, 32 x 32, 128 x 32)
 #define TAGI_GEMM_COMBOS_SHARED_B_BNF(X)                                                 \
   X(PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4)
-static inline bool bnf_cfg(int cfg) { return cfg == 3 || cfg == 4 || cfg == 5; }
+static inline bool bnf_cfg(int cfg) { return cfg >= 3; }
 // The Linear parameter-delta loader pairs that also get the in-place update (EPI 2), in
 // every tile config
 #define TAGI_GEMM_COMBOS_SHARED_A_UPD(X)                                                 \
@@ -1994,22 +2395,64 @@ static inline bool bnf_cfg(int cfg) { return cfg == 3 || cfg == 4 || cfg == 5; }
 #define TAGI_GEMM_COMBOS_FWD_RELU(X)                                                     \
   X(PROD_FWD, LD_STR_K4, LD_STR_MN4) X(PROD_FWD, LD_STR_K_S, LD_STR_MN_S)
 #define TAGI_GEMM_COMBOS_SHARED_A_RELU(X)                                                \
-  X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4) X(PROD_SHARED_A, LD_STR_MN_S, LD_STR_MN_S)
+  X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4) X(PROD_SHARED_A, LD_STR_K_S, LD_STR_MN_S)
 
+// The split kernel's combinations (the batched products stay with the fp32 kernel, whose
+// bits the fused attention kernels repeat)
+#define TAGI_GEMM_SPLIT_FWD(X)                                                           \
+  X(PROD_FWD, LD_CFWD_A4T, LD_CFWD_B4T, 0) X(PROD_FWD, LD_CFWD_A4, LD_CFWD_B4, 0)        \
+  X(PROD_FWD, LD_CFWD_A_S, LD_CFWD_B4, 0) X(PROD_FWD, LD_CFWD_A_S, LD_CFWD_B4U, 0)       \
+  X(PROD_FWD, LD_STR_K4, LD_STR_MN4, 0) X(PROD_FWD, LD_STR_K4U, LD_STR_MN4U, 0)          \
+  X(PROD_FWD, LD_STR_K4, LD_STR_MN4, 4) X(PROD_FWD, LD_STR_K4U, LD_STR_MN4U, 4)
+#define TAGI_GEMM_SPLIT_SHARED_B(X)                                                      \
+  X(PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 0) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 0) \
+  X(PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 1) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 1) \
+  X(PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T, 3) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4, 3) \
+  X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B4, 0) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_B4U, 0) \
+  X(PROD_SHARED_B, LD_CBWD_A_S, LD_CBWD_B4U, 0)                                          \
+  X(PROD_SHARED_B, LD_STR_K4, LD_STR_K4, 0) X(PROD_SHARED_B, LD_STR_K4U, LD_STR_K4U, 0)
+#define TAGI_GEMM_SPLIT_SHARED_A(X)                                                      \
+  X(PROD_SHARED_A, LD_CWG_A4T, LD_STR_MN4, 0) X(PROD_SHARED_A, LD_CWG_A4, LD_STR_MN4, 0) \
+  X(PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN4, 0) X(PROD_SHARED_A, LD_CWG_A_S, LD_STR_MN4U, 0) \
+  X(PROD_SHARED_A, LD_STR_MN4, LD_STR_MN4, 0) X(PROD_SHARED_A, LD_STR_MN4U, LD_STR_MN4U, 0) \
+  X(PROD_SHARED_A, LD_STR_MN4, LD_STR_MN4, 2) X(PROD_SHARED_A, LD_STR_MN4U, LD_STR_MN4U, 2) \
+  X(PROD_SHARED_A, LD_CFWD_A4T, LD_CFWD_B4T, 0) X(PROD_SHARED_A, LD_CFWD_A4, LD_CFWD_B4, 0) \
+  X(PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B4, 0) X(PROD_SHARED_A, LD_CFWD_A_S, LD_CFWD_B4U, 0) \
+  X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4, 0) X(PROD_SHARED_A, LD_STR_K4U, LD_STR_MN4U, 0) \
+  X(PROD_SHARED_A, LD_STR_K4, LD_STR_MN4, 4) X(PROD_SHARED_A, LD_STR_K4U, LD_STR_MN4U, 4)
+
+// (defined in tagi_gemm_split.h)
 template <int PROD, class CFG, int KA, int KB, int EPI = 0>
-void launch_cfg(const GemmArgs& g, int64_t grid_x, int64_t grid_y, hipStream_t s)
-#ifdef TAGI_GEMM_DEFINE_LAUNCH
-{
-  hipLaunchKernelGGL((gemm_kernel<PROD, CFG, KA, KB, EPI>), dim3((unsigned)grid_x, (unsigned)grid_y), dim3(CFG::NTH),
-                     0, s, g);
+void launch_cfg(const GemmArgs& g, int64_t grid_x, int64_t grid_y, hipStream_t s);
+
+// The split kernel's launch (cfg: a split tile config). The tile-aligned conv kinds need
+// 32-wide k tiles within a tap (or image); where only 16-wide ones are, the general kinds run.
+constexpr int any_kind(int k) {  // float4 kinds for rows of any alignment in place of scalar ones
+  return k == LD_STR_K_S ? LD_STR_K4U : k == LD_STR_MN_S ? LD_STR_MN4U : k == LD_CFWD_B_S ? LD_CFWD_B4U
+         : k == LD_CBWD_B_S ? LD_CBWD_B4U : k;
 }
-#else
-    ;
-#endif
+constexpr int untiled_kind(int k) {
+  return k == LD_CFWD_A4T ? LD_CFWD_A4 : k == LD_CFWD_B4T ? LD_CFWD_B4 : k == LD_CBWD_A4T ? LD_CBWD_A4
+         : k == LD_CBWD_BK4T ? LD_CBWD_BK4 : k == LD_CWG_A4T ? LD_CWG_A4 : k;
+}
+
+template <int PROD, int KA, int KB, int EPI>
+static inline void launch_split(int cfg, const GemmArgs& g, int64_t gx, int64_t gy, hipStream_t s) {
+  switch (cfg) {
+    case 6: launch_cfg<PROD, X256x128, KA, KB, EPI>(g, gx, gy, s); break;
+    case 7: launch_cfg<PROD, X256x64, KA, KB, EPI>(g, gx, gy, s); break;
+    case 8: launch_cfg<PROD, X128x128, KA, KB, EPI>(g, gx, gy, s); break;
+    case 9: launch_cfg<PROD, X128x64, KA, KB, EPI>(g, gx, gy, s); break;
+    case 10: launch_cfg<PROD, X64x64, KA, KB, EPI>(g, gx, gy, s); break;
+    case 11: launch_cfg<PROD, X128x32, KA, KB, EPI>(g, gx, gy, s); break;
+    case 12: launch_cfg<PROD, X64x32, KA, KB, EPI>(g, gx, gy, s); break;
+    default: launch_cfg<PROD, X32x32, KA, KB, EPI>(g, gx, gy, s); break;
+  }
+}
 
 // Launch with plan p. For phased (conv input-delta) launches grid_x covers the largest
 // phase and blocks past a phase's tiles exit at once.
-template <int PROD, int KA, int KB, int EPI = 0>
+template <int PROD, int KA, int KB, int EPI = 0, int XD = XD_NONE>
 static inline int run_gemm(GemmArgs g, int64_t batch, const Plan& p, float* ws, int64_t ws_bytes, hipStream_t s,
                            const char* what, int64_t grid_x_override = 0) {
   if constexpr (EPI == 1 || EPI == 3)
@@ -2035,7 +2478,19 @@ static inline int run_gemm(GemmArgs g, int64_t batch, const Plan& p, float* ws, 
   const int64_t gy = batch * p.splits;
   TAGI_REQUIRE(gx > 0 && gx < (1ll << 31) && gy < 65536, "%s: grid out of range (%lld x %lld)", what, (long long)gx,
                (long long)gy);
-  if constexpr (EPI == 1 || EPI == 3) {
+  if (p.cfg >= kNumCfg32) {
+    if constexpr (XD != XD_NONE) {
+      TAGI_REQUIRE(p.xd == XD && (p.splits == 1 || p.k_chunk % 32 == 0), "%s: internal: plan of another call", what);
+      // EPI 2 and 4 apply their epilogue in the kernel only when unsplit, as below
+      constexpr int E0 = (EPI == 2 || EPI == 4) ? 0 : EPI;
+      constexpr int NA = any_kind(KA), NB = any_kind(KB), UA = untiled_kind(KA), UB = untiled_kind(KB);
+      if (UA != KA && !g.tile32) launch_split<PROD, UA, UB, E0>(p.cfg, g, gx, gy, s);
+      else if (E0 != EPI && p.splits > 1) launch_split<PROD, NA, NB, E0>(p.cfg, g, gx, gy, s);
+      else launch_split<PROD, NA, NB, EPI>(p.cfg, g, gx, gy, s);
+    } else {
+      return fail(TAGI_ERR_ARG, "%s: internal: no split kernel for this product", what);
+    }
+  } else if constexpr (EPI == 1 || EPI == 3) {
     switch (p.cfg) {
       case 3: launch_cfg<PROD, C64x64, KA, KB, EPI>(g, gx, gy, s); break;
       case 5: launch_cfg<PROD, C128x32, KA, KB, EPI>(g, gx, gy, s); break;

@@ -61,8 +61,8 @@ extern "C" int tagi_linear_fwd_noalloc(const float* ma, const float* Sa, const f
   int rc = linear_fwd_check(what, ma, Sa, mw, Sw, Sz, M, K, N);
   if (rc != TAGI_OK) return rc;
   // the plan tagi_linear_fwd runs with its full workspace, so results are the same bits
-  const Plan p = linear_fwd_plan(M, K, N);
-  const int64_t need = plan_ws_bytes(p, M, N, 1);
+  const Plan p = linear_fwd_plan(M, K, N), p32 = linear_fwd_plan32(M, K, N);
+  const int64_t need32 = plan_ws_bytes(p32, M, N, 1), need = need32 > plan_ws_bytes(p, M, N, 1) ? need32 : plan_ws_bytes(p, M, N, 1);
   TAGI_REQUIRE(need <= (int64_t)TAGI_LINEAR_FWD_NOALLOC_SCRATCH_BYTES,
                "%s: M=%lld K=%lld N=%lld needs %lld bytes of split-K scratch, above the fixed %lld; use "
                "tagi_linear_fwd with a workspace",
