@@ -29,8 +29,9 @@ def inputs(shape, gen, scale=1.0):
 
 # widths 4 and up, one under and over the 16/32/64/128 tile sides and the 32-wide k tiles,
 # rows of every alignment, reductions of one tile and of many
-LINEAR = [(1, 5, 4), (64, 32, 64), (63, 31, 65), (130, 33, 127), (257, 100, 129), (1000, 255, 61), (31, 4096, 1030),
-          (515, 517, 1027), (2050, 64, 516), (96, 2052, 700), (4099, 7, 9)]
+LINEAR = [(1, 5, 4), (64, 32, 64), (4095, 31, 1025), (8130, 33, 127), (2057, 100, 1029), (40001, 255, 61),
+          (31, 4096, 1030), (515, 517, 1027), (2050, 64, 516), (96, 2052, 700), (99999, 39, 11), (16385, 7, 769),
+          (769, 50001, 4), (5, 2048, 8193)]
 
 
 @pytest.mark.parametrize("M,K,N", LINEAR)
@@ -63,8 +64,8 @@ def test_linear(M, K, N):
 
 # channels in and out of every alignment, taps that straddle k tiles, one-tap kernels, strides,
 # images whose pixels do not fill a k tile
-CONV = [(3, 32, 8, 64, 3, 1), (5, 48, 9, 80, 3, 1), (2, 13, 11, 38, 5, 1), (9, 37, 7, 5, 3, 2), (4, 64, 16, 17, 1, 1),
-        (2, 5, 32, 66, 3, 1), (16, 30, 8, 4, 3, 2), (7, 96, 4, 33, 2, 2)]
+CONV = [(3, 32, 8, 64, 3, 1), (33, 64, 17, 80, 3, 1), (29, 13, 31, 138, 5, 1), (97, 37, 27, 65, 3, 2), (64, 64, 31, 17, 1, 1),
+        (55, 5, 32, 66, 3, 1), (116, 30, 28, 70, 3, 2), (57, 96, 14, 133, 2, 2), (32, 32, 32, 48, 3, 1), (40, 48, 16, 96, 5, 2)]
 
 
 @pytest.mark.parametrize("B,C,H,Cout,k,s", CONV)
@@ -96,7 +97,7 @@ def test_conv(B, C, H, Cout, k, s):
     check(layer.delta_Sw, Vw**2 * wgr(a**2, e), Vw**2 * wgr(a**2, e.abs()), M, 3, "delta_Sw")
 
 
-@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (300, 100, 130), (130, 700, 1001)])
+@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (3000, 100, 1130), (130, 700, 1001)])
 def test_infinities_and_nan(M, K, N):
     """One infinite, one NaN and one huge operand: the outputs they reach are those of fp32
     arithmetic, the others are as without them."""

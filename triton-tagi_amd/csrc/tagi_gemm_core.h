@@ -2137,19 +2137,23 @@ struct Plan {
 
 // Whether a product with a split kernel runs it (else the fp32 kernel). The split kernel is
 // the faster one wherever the matrix cores or the loads' volume bound the launch, 1.2 to 1.8
-// times at 2^28 multiply-adds and more, and no slower on small products with a short
-// reduction (their k tiles are twice as long, so there are half as many). Not on
-//   * few multiply-adds over a long reduction, which both kernels cut into many splits whose
-//     chains of loads and barriers are the time: the fp32 kernel's 16-wide k tiles give the
-//     shorter chain (256 x 784 x 256 forward 15.5 against 16.5 us, its parameter deltas 13.8
-//     against 14.7; 128 x 1024 x 256 14.1 against 14.7);
-//   * element-wise patches under one k tile (a 3-channel 3 x 3 input at 131072 pixels: 28.9
-//     against 33.3 us);
+// times at 2^28 multiply-adds and more. Not on
+//   * products whose launch, loads' latency and barriers are the time: under 2^25
+//     multiply-adds (the kernels tie within 2 us when repeated, but the split kernel's longer
+//     code is fetched anew in a step of many kernels: MLP steps of batch 42 and 72 2-4%
+//     slower), and under 2^26 over a reduction of 256 and more, where the fp32 kernel's
+//     16-wide k tiles give the shorter chain (256 x 784 x 256 forward 15.5 against 16.5 us,
+//     its parameter deltas 13.8 against 14.7);
+//   * element-wise patches, whose decode is the time in both: under one k tile (a 3-channel 3 x
+//     3 input at 131072 pixels 28.9 against 33.3 us), and input deltas of more than 64
+//     channels (137 <- 362 channels, stride 2, with its other products 256 against 290; 42 <-
+//     70 channels 44.5 against 40.5);
 //   * sides under 4, which its float4 loads of any alignment do not cover.
-static inline bool use_split(int64_t R, int64_t C, int64_t Kred, int64_t batch, int xd, bool narrow) {
+static inline bool use_split(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, int xd, bool narrow) {
   if (xd == XD_NONE || narrow) return false;
-  if (Kred >= 256 && (double)R * C * Kred * batch < (double)(1 << 26)) return false;
-  return !((xd & XD_SCALAR) && Kred < 32);
+  const double macs = (double)R * C * Kred * batch;
+  if (macs < (double)(1 << 25) || (Kred >= 256 && macs < (double)(1 << 26))) return false;
+  return !(xd & XD_SCALAR) || (prod == PROD_SHARED_B ? C <= 64 : Kred >= 32);
 }
 
 // The split kernel's plan, from the same kind of model as the fp32 kernel's below: blocks run
@@ -2204,6 +2208,10 @@ static inline Plan choose_split_plan(int64_t R, int64_t C, int64_t Kred, int64_t
         blocks = (int64_t)ceil(eq);
       }
       double block_s = (2.0 * BM * BN * kc * products) / (peak_cu * kEff[x][prod]) + BM * BN * kOut;
+      // parameter deltas applied by one block per CU: its epilogue loads every output's
+      // variance with nothing beside it to hide them (4097 x 11008 over 256: 489 us in 256 x
+      // 128 tiles, 423 in 64 x 64)
+      if (bpc == 1 && actual == 1 && side == XD_B) block_s += BM * BN * 1.0e-9;
       if (xd & XD_SCALAR) block_s += kCfg[ci].BM * (double)kc * kDecode;
       const double chain = kFixed + (double)(kc / 32) * kChain[x][prod];
       auto round_s = [&](double r) {
@@ -2272,7 +2280,7 @@ static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int6
   double best_t = DBL_MAX;
   const double peak_cu = 157.3e12 / 256.0;
   const int64_t max_sp = allow_split ? (max_splits < 512 ? max_splits : 512) : 1;
-  if (use_split(R, C, Kred, batch, xd, narrow)) return choose_split_plan(R, C, Kred, batch, prod, max_sp, phase_k, xd);
+  if (use_split(R, C, Kred, batch, prod, xd, narrow)) return choose_split_plan(R, C, Kred, batch, prod, max_sp, phase_k, xd);
   for (int ci = 0; ci < kNumCfg32; ++ci) {
     const int BM = kCfg[ci].BM, BN = kCfg[ci].BN;
     const int64_t tm = cdiv(R, BM), tn = cdiv(C, BN);
