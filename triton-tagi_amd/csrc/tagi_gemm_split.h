@@ -19,8 +19,8 @@
 // MFMAs, which sustain 2.1 PF/s here where 32x32x16 throttles at 1.85 (random operands).
 // Measured with the fp32 kernel's best tile on the left (4096 x 4096 x 4096): forward 2984 ->
 // 1929 us (214 TF/s of fp32 products), input deltas 1964 -> 1231, parameter deltas 2225 ->
-// 1540; a 64-channel 3 x 3 Conv2D at 131072 pixels: forward 236 -> 162, input deltas 172 ->
-// 131, parameter deltas 183 -> 151.
+// 1540; a 64-channel 3 x 3 Conv2D at 131072 pixels: forward 254 -> 191, input deltas 184 ->
+// 140, parameter deltas 184 -> 155 (one run; the layer 584 -> 487).
 #pragma once
 #include "tagi_gemm_core.h"
 
@@ -195,34 +195,45 @@ __global__ void __launch_bounds__(X::NTH, (split_minw<PROD, X, KA, KB>())) gemm_
   };
   const int lrow = q * QS + phys(rl) * 16;  // the lane's 16 bytes of staged fragment 0
 
-  auto product = [&](auto P, const unsigned char* buf, float sg, auto&& after) {
-    uintx4 fd[TD][3];
+  // Products P .. P + N - 1 of one k tile (N 2: the forward's two variance products, whose
+  // partial sums share one chain and one addition)
+  auto product = [&](auto P, auto N, const unsigned char* buf, float sg, auto&& after) {
+    constexpr int n_ = decltype(N)::value;
+    uintx4 fd[n_][TD][3];
+    static_for<0, n_>([&](auto n) {
+      using Q = std::integral_constant<int, decltype(P)::value + decltype(n)::value>;
 #pragma unroll
-    for (int f = 0; f < TD; ++f)
+      for (int f = 0; f < TD; ++f)
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        uint32_t h, m, l;
-        split_pair(dval(P, f, e), dval(P, f, e + 1), h, m, l);
-        fd[f][0][e / 2] = h;
-        fd[f][1][e / 2] = m;
-        fd[f][2][e / 2] = l;
-      }
+        for (int e = 0; e < 8; e += 2) {
+          uint32_t h, m, l;
+          split_pair(dval(Q{}, f, e), dval(Q{}, f, e + 1), h, m, l);
+          fd[n][f][0][e / 2] = h;
+          fd[n][f][1][e / 2] = m;
+          fd[n][f][2][e / 2] = l;
+        }
+    });
     after();
 #pragma unroll
     for (int j = 0; j < TL; ++j) {
-      uintx4 fl[3];
+      uintx4 fl[n_][3];
 #pragma unroll
-      for (int s = 0; s < 3; ++s) fl[s] = *reinterpret_cast<const uintx4*>(buf + lrow + (P * 3 + s) * PS + j * 256);
+      for (int n = 0; n < n_; ++n)
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          fl[n][s] = *reinterpret_cast<const uintx4*>(buf + lrow + ((P + n) * 3 + s) * PS + j * 256);
       floatx4 t[TD];
 #pragma unroll
       for (int f = 0; f < TD; ++f) t[f] = floatx4{0.f, 0.f, 0.f, 0.f};
-      // smallest products first, so that each addition loses the least
+      // smallest part products first, so that each addition loses the least
       constexpr int sd[6] = {0, 2, 1, 0, 1, 0}, sl[6] = {2, 0, 1, 1, 0, 0};
 #pragma unroll
       for (int c = 0; c < 6; ++c)
 #pragma unroll
-        for (int f = 0; f < TD; ++f)
-          t[f] = DA ? mfma_bf16(fd[f][sd[c]], fl[sl[c]], t[f]) : mfma_bf16(fl[sl[c]], fd[f][sd[c]], t[f]);
+        for (int n = 0; n < n_; ++n)
+#pragma unroll
+          for (int f = 0; f < TD; ++f)
+            t[f] = DA ? mfma_bf16(fd[n][f][sd[c]], fl[n][sl[c]], t[f]) : mfma_bf16(fl[n][sl[c]], fd[n][f][sd[c]], t[f]);
 #pragma unroll
       for (int f = 0; f < TD; ++f) {
         floatx4& a = acc[P == 0 ? 0 : 1][DA ? f : j][DA ? j : f];
@@ -234,6 +245,14 @@ __global__ void __launch_bounds__(X::NTH, (split_minw<PROD, X, KA, KB>())) gemm_
       if (j % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
   };
+  // The forward's variance products share a chain in the 256 x 64 tiles: a quarter fewer VALU
+  // additions (residual block 988 -> 969 us, 64-channel 3 x 3 layer 490 -> 483). In the wider
+  // tiles the second set of fragments does not fit the registers, and in the others, and
+  // beside element-wise or unaligned loaders, it gains nothing (42 -> 70 channels 119.3 ->
+  // 120.1).
+  constexpr bool JOIN = PROD == PROD_FWD && NW == 8 && DM == 32 && LM == 64 && KindTraits<KA>::vec4 &&
+                        !KindTraits<KA>::any && !KindTraits<KB>::any;
+  constexpr int NPASS = JOIN ? 2 : NP;
 
   if (nk > 0) {
     ls.fetch(os, z, l0, kbeg);
@@ -251,12 +270,12 @@ __global__ void __launch_bounds__(X::NTH, (split_minw<PROD, X, KA, KB>())) gemm_
     const unsigned char* buf = smem + (NBUF == 2 ? (t & 1) * BUF : 0);
     if constexpr (NBUF == 1) ls.fetch(os, z, l0, k0 + BK);
     ld.settle(od, d0, k0);
-    static_for<0, NP>([&](auto P) {
-      if constexpr (NBUF == 2 && P == NP - 2) ls.fetch(os, z, l0, k0 + BK);
-      product(P, buf, sign(t), [&] {
-        if constexpr (P == NP - 1) ld.fetch(od, z, d0, k0 + BK);
+    static_for<0, NPASS>([&](auto P) {
+      if constexpr (NBUF == 2 && P == NPASS - 2) ls.fetch(os, z, l0, k0 + BK);
+      product(P, std::integral_constant<int, (JOIN && P == 1) ? 2 : 1>{}, buf, sign(t), [&] {
+        if constexpr (P == NPASS - 1) ld.fetch(od, z, d0, k0 + BK);
       });
-      if constexpr (NBUF == 2 && P == NP - 2) {
+      if constexpr (NBUF == 2 && P == NPASS - 2) {
         ls.settle(os, l0, k0 + BK);
         stage(smem + ((t + 1) & 1) * BUF, t + 1);
       }
