@@ -91,7 +91,23 @@ int tagi_probe_stream(const float* src, float* dst, int64_t n, int64_t blocks, i
 int tagi_probe_stream_variant(const float* src, float* dst, int64_t n, int64_t dst_n, int64_t blocks, int mode,
                               int unroll, int flags, tagi_stream_t stream);
 
+/* The launch that a Linear or Conv2D product gets (no counterpart in the reference; host
+ * only, for tests and tools): whether the split-operand kernel runs it (else the fp32-MFMA
+ * kernel), the rows and columns of a block's tile, the tiles along both (of the largest
+ * stride phase), and the reduction's splits of k_chunk each. op is a TAGI_OP_*; ws_bytes is
+ * the workspace that the call is given for partial sums, -1 for as much as it asks for. */
+typedef struct {
+  int64_t split_kernel, tile_rows, tile_cols, tiles_rows, tiles_cols, splits, k_chunk;
+} tagi_plan;
+enum {
+  TAGI_OP_FWD = 0,       /* forward */
+  TAGI_OP_FWD_FIXED = 1, /* forward of an input without variance (Sa NULL) */
+  TAGI_OP_BWD_DELTA = 2, /* input deltas */
+  TAGI_OP_WGRAD = 3      /* parameter deltas, with the bias */
+};
+
 /* ------------------------------------------------------------------ Linear ---- */
+int tagi_linear_plan(int op, int64_t M, int64_t K, int64_t N, int64_t ws_bytes, tagi_plan* out);
 /* Fused Linear forward moments, one MFMA pass sharing the A/B tiles:
  *   mz = ma @ mw + mb
  *   Sz = ma^2 @ Sw + Sa @ (mw^2 + Sw) + Sb
@@ -304,6 +320,9 @@ int tagi_attn_score_deltas_qk_joint(const float* d_mu, const float* d_var, int64
 typedef struct {
   int64_t N, C, H, W, Cout, k, stride, pad_top, pad_left, Ho, Wo;
 } tagi_conv_geom;
+
+/* The launch that a Conv2D product gets, as tagi_linear_plan. */
+int tagi_conv2d_plan(int op, const tagi_conv_geom* g, int64_t ws_bytes, tagi_plan* out);
 
 /* Implicit-GEMM forward: patches are gathered into LDS, never materialised.
  *   mz = P(ma) @ mw + mb ; Sz = P(ma)^2 @ Sw + P(Sa) @ (mw^2 + Sw) + Sb (channels-last).

@@ -79,3 +79,29 @@ def test_noalloc_refuses_shapes_beyond_the_scratch(dev):
     rc = lib.tagi_linear_fwd_noalloc(*([fake] * 8), M, K, N, torch.cuda.current_stream(dev).cuda_stream)
     assert rc == _lib.TAGI_ERR_ARG if hasattr(_lib, "TAGI_ERR_ARG") else rc == 1
     assert "scratch" in _lib.last_error()
+
+
+@pytest.mark.parametrize("M,K,N", [(4097, 4096, 4097), (512, 2048, 50257)])
+def test_forward_with_partial_planes_larger_than_the_scratch(dev, M, K, N):
+    """One pair of partial planes is above the scratch: the forward runs unsplit, with a
+    workspace, without allocation and with the ReLU folded in."""
+    from triton_tagi_amd import _lib
+
+    host = _inputs(M, K, N, 3)
+    t = [x.to(dev) for x in host]
+    ws = torch.empty(_lib.query("tagi_linear_fwd_ws_bytes", M, K, N) // 4 + 1, device=dev)
+    ref_m, ref_S = _call("tagi_linear_fwd", dev, t, M, K, N, ws)
+    got_m, got_S = _call("tagi_linear_fwd_noalloc", dev, t, M, K, N)
+    assert torch.equal(got_m, ref_m) and torch.equal(got_S, ref_S)
+    out = [torch.empty(M, N, device=dev) for _ in range(3)]
+    st = torch.cuda.current_stream(dev).cuda_stream
+    _lib.call("tagi_linear_fwd_relu", *[x.data_ptr() for x in t + out], M, K, N, ws.data_ptr(), ws.numel() * 4, st)
+    rel = [torch.empty(M, N, device=dev) for _ in range(3)]
+    _lib.call("tagi_relu_fwd", ref_m.data_ptr(), ref_S.data_ptr(), *[x.data_ptr() for x in rel], M * N, st)
+    assert all(torch.equal(a, b) for a, b in zip(out, rel))
+    rows, cols = torch.arange(0, M, M // 50), torch.arange(0, N, N // 50)
+    a, S, mw, Sw, mb, Sb = (x.double() for x in host)
+    rm, rS = O.linear_moments(a[rows], S[rows], mw[:, cols], Sw[:, cols], mb[:, cols], Sb[:, cols])
+    assert_scaled_close(got_m[rows][:, cols], rm, a[rows].abs() @ mw[:, cols].abs() + mb[:, cols].abs(),
+                        1e-5, 1e-6, "mz sample")
+    assert_scaled_close(got_S[rows][:, cols], rS, None, 1e-5, 1e-6, "Sz sample")

@@ -101,9 +101,34 @@ static Plan conv_bwd_plan(const tagi_conv_geom* g, bool split = true) {
 }
 
 // rows: the weight rows (c, kh, kw), plus the ones row of the bias sums when the GEMM forms them
-static Plan conv_wgrad_plan(const tagi_conv_geom* g, bool bias) {
-  return choose_plan(g->C * g->k * g->k + (bias ? 1 : 0), g->Cout, g->N * g->Ho * g->Wo, 1, PROD_SHARED_A, true, 512, nullptr, XD_B,
-                     g->Cout < 4);
+static Plan conv_wgrad_plan(const tagi_conv_geom* g, bool bias, bool split = true) {
+  return choose_plan(g->C * g->k * g->k + (bias ? 1 : 0), g->Cout, g->N * g->Ho * g->Wo, 1, PROD_SHARED_A, split,
+                     split ? 512 : 1, nullptr, XD_B, g->Cout < 4);
+}
+
+extern "C" int tagi_conv2d_plan(int op, const tagi_conv_geom* g, int64_t ws_bytes, tagi_plan* out) {
+  const char* what = "tagi_conv2d_plan";
+  int rc = check_geom(g, what);
+  if (rc) return rc;
+  TAGI_REQUIRE(out, "%s: null pointer", what);
+  TAGI_REQUIRE(op >= TAGI_OP_FWD && op <= TAGI_OP_WGRAD, "%s: bad product %d", what, op);
+  auto plan = [&](bool split) {
+    return op == TAGI_OP_BWD_DELTA ? conv_bwd_plan(g, split)
+           : op == TAGI_OP_WGRAD   ? conv_wgrad_plan(g, true, split)
+                                   : conv_fwd_plan(g, op == TAGI_OP_FWD_FIXED, split);
+  };
+  int64_t R = g->N * g->Ho * g->Wo, C = g->Cout, batch = 1, K;
+  if (op == TAGI_OP_BWD_DELTA) {
+    bwd_phase0(g, &R, &K);
+    C = g->C;
+    batch = g->stride * g->stride;
+  } else if (op == TAGI_OP_WGRAD) {
+    R = g->C * g->k * g->k + 1;
+  }
+  Plan p = plan(true);
+  if (ws_bytes >= 0 && ws_bytes < plan_ws_bytes(p, R, C, batch)) p = plan(false);
+  *out = plan_info(p);
+  return TAGI_OK;
 }
 
 static int64_t wt_floats(const tagi_conv_geom* g) { return ((g->C * g->k * g->k * g->Cout) + 3) / 4 * 4; }
@@ -479,7 +504,7 @@ extern "C" int tagi_conv2d_wgrad(const float* ma, const float* dmz, const float*
   a.Kred = (int)M;
   Plan p = conv_wgrad_plan(g, bias);
   if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, a.R, N, 1)))
-    p = choose_plan(a.R, N, M, 1, PROD_SHARED_A, false, 1, nullptr, XD_B, N < 4);
+    p = conv_wgrad_plan(g, bias, false);
   p.tiles_m = (int)cdiv(a.R, cfg_bm(p.cfg, p.xd));
   const bool va = g->C % 4 == 0 && al16(ma);
   const bool vb = g->Cout % 4 == 0 && al16(dmz) && al16(dSz);

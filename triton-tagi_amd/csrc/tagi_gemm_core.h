@@ -2279,7 +2279,8 @@ static inline Plan choose_plan_uncached(int64_t R, int64_t C, int64_t Kred, int6
   Plan best{3, 1, (int)Kred, 1, 1, XD_NONE};
   double best_t = DBL_MAX;
   const double peak_cu = 157.3e12 / 256.0;
-  const int64_t max_sp = allow_split ? (max_splits < 512 ? max_splits : 512) : 1;
+  // at least the unsplit plan is tried, so that no search comes back empty
+  const int64_t max_sp = !allow_split || max_splits < 1 ? 1 : max_splits < 512 ? max_splits : 512;
   if (use_split(R, C, Kred, batch, prod, xd, narrow)) return choose_split_plan(R, C, Kred, batch, prod, max_sp, phase_k, xd);
   for (int ci = 0; ci < kNumCfg32; ++ci) {
     const int BM = kCfg[ci].BM, BN = kCfg[ci].BN;
@@ -2358,6 +2359,11 @@ static inline Plan choose_plan(int64_t R, int64_t C, int64_t Kred, int64_t batch
 
 static inline int64_t plan_ws_bytes(const Plan& p, int64_t R, int64_t C, int64_t batch) {
   return p.splits > 1 ? (int64_t)p.splits * 2 * R * C * batch * (int64_t)sizeof(float) : 0;
+}
+
+static inline tagi_plan plan_info(const Plan& p) {
+  return tagi_plan{p.cfg >= kNumCfg32 ? 1 : 0, cfg_bm(p.cfg, p.xd), cfg_bn(p.cfg, p.xd), p.tiles_m, p.tiles_n, p.splits,
+                   p.k_chunk};
 }
 
 // The (product, tile config, loader) combinations the entry points launch. Each
@@ -2471,6 +2477,8 @@ static inline int run_gemm(GemmArgs g, int64_t batch, const Plan& p, float* ws, 
                    g.b.nbytes < (int64_t)kBufOutOfRange,
                "%s: an operand spans %lld / %lld bytes; at most 2 GiB per operand", what, (long long)g.a.nbytes,
                (long long)g.b.nbytes);
+  TAGI_REQUIRE(p.splits >= 1 && p.tiles_m >= 1 && p.tiles_n >= 1 && (int64_t)p.splits * p.k_chunk >= g.Kred,
+               "%s: internal: the plan does not cover the product", what);
   g.tiles_m = p.tiles_m;
   g.tiles_n = p.tiles_n;
   g.splits = p.splits;

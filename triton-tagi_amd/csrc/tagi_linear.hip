@@ -12,20 +12,48 @@ static bool linear_narrow(int64_t K, int64_t N) { return K < 4 || N < 4; }
 // accepts is decided by its workspace.
 Plan tagi::linear_fwd_plan32(int64_t M, int64_t K, int64_t N) { return choose_plan(M, N, K, 1, PROD_FWD, true, 16); }
 
-Plan tagi::linear_fwd_plan(int64_t M, int64_t K, int64_t N) {
-  const Plan p = choose_plan(M, N, K, 1, PROD_FWD, true, 16, nullptr, XD_A, linear_narrow(K, N));
+// split: whether the reduction may be cut (the caller's workspace holds the partial sums)
+Plan tagi::linear_fwd_plan(int64_t M, int64_t K, int64_t N, bool split) {
+  const Plan p = choose_plan(M, N, K, 1, PROD_FWD, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
   constexpr int64_t kScratch = TAGI_LINEAR_FWD_NOALLOC_SCRATCH_BYTES;
   if (plan_ws_bytes(p, M, N, 1) <= kScratch || plan_ws_bytes(linear_fwd_plan32(M, K, N), M, N, 1) > kScratch) return p;
-  // the fixed scratch holds every shape that tagi_linear_fwd_noalloc accepts: fewer splits
-  return choose_plan(M, N, K, 1, PROD_FWD, true, kScratch / (8 * M * N), nullptr, XD_A, linear_narrow(K, N));
+  // the fixed scratch holds every shape that tagi_linear_fwd_noalloc accepts: fewer splits,
+  // none where one pair of partial planes is already larger (M N > 2^24)
+  const int64_t fit = kScratch / (8 * M * N);
+  return choose_plan(M, N, K, 1, PROD_FWD, fit > 1, fit > 1 ? fit : 1, nullptr, XD_A, linear_narrow(K, N));
 }
-static Plan linear_bwd_plan(int64_t M, int64_t K, int64_t N) { return choose_plan(M, K, N, 1, PROD_SHARED_B, true, 16, nullptr, XD_A, linear_narrow(K, N)); }
-static Plan linear_wgrad_plan(int64_t M, int64_t K, int64_t N) { return choose_plan(K + 1, N, M, 1, PROD_SHARED_A, true, 512, nullptr, XD_B, linear_narrow(K, N)); }
+static Plan linear_bwd_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
+  return choose_plan(M, K, N, 1, PROD_SHARED_B, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
+}
+static Plan linear_wgrad_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
+  return choose_plan(K + 1, N, M, 1, PROD_SHARED_A, split, split ? 512 : 1, nullptr, XD_B, linear_narrow(K, N));
+}
 
 // A deterministic input (no variance, Sa NULL): mean = ma mw, variance = ma^2 Sw, the
 // shared-A product (two MFMAs per k-step instead of three; the terms Sa (mw^2 + Sw) it
 // leaves out are exact zeros)
-static Plan linear_fwd0_plan(int64_t M, int64_t K, int64_t N) { return choose_plan(M, N, K, 1, PROD_SHARED_A, true, 16, nullptr, XD_A, linear_narrow(K, N)); }
+static Plan linear_fwd0_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
+  return choose_plan(M, N, K, 1, PROD_SHARED_A, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
+}
+
+extern "C" int tagi_linear_plan(int op, int64_t M, int64_t K, int64_t N, int64_t ws_bytes, tagi_plan* out) {
+  const char* what = "tagi_linear_plan";
+  TAGI_REQUIRE(out, "%s: null pointer", what);
+  TAGI_REQUIRE(M > 0 && K > 0 && N > 0, "%s: sizes must be positive", what);
+  TAGI_REQUIRE(fits_i32(M * K) && fits_i32((K + 1) * N) && fits_i32(M * N), "%s: too large for 32-bit tiles", what);
+  auto plan = [&](bool split) {
+    return op == TAGI_OP_FWD         ? linear_fwd_plan(M, K, N, split)
+           : op == TAGI_OP_FWD_FIXED ? linear_fwd0_plan(M, K, N, split)
+           : op == TAGI_OP_BWD_DELTA ? linear_bwd_plan(M, K, N, split)
+                                     : linear_wgrad_plan(M, K, N, split);
+  };
+  TAGI_REQUIRE(op >= TAGI_OP_FWD && op <= TAGI_OP_WGRAD, "%s: bad product %d", what, op);
+  const int64_t R = op == TAGI_OP_WGRAD ? K + 1 : M, C = op == TAGI_OP_BWD_DELTA ? K : N;
+  Plan p = plan(true);
+  if (ws_bytes >= 0 && ws_bytes < plan_ws_bytes(p, R, C, 1)) p = plan(false);
+  *out = plan_info(p);
+  return TAGI_OK;
+}
 
 extern "C" int64_t tagi_linear_fwd_ws_bytes(int64_t M, int64_t K, int64_t N) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
@@ -75,7 +103,7 @@ static int linear_fwd0(const char* what, const float* ma, const float* mw, const
   TAGI_REQUIRE(fits_i32(M * K) && fits_i32(K * N) && fits_i32(M * N), "%s: too large for 32-bit tiles", what);
   Plan p = linear_fwd0_plan(M, K, N);
   if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, M, N, 1)))
-    p = choose_plan(M, N, K, 1, PROD_SHARED_A, false, 1, nullptr, XD_A, linear_narrow(K, N));
+    p = linear_fwd0_plan(M, K, N, false);
   ProfScope ps(FAM_LINEAR_FWD, s, 2.0 * 2 * M * K * N, 4.0 * (M * K + 2 * K * N + (relu_J ? 3 : 2) * M * N));
   GemmArgs g{};
   g.a = strided_operand(ma, nullptr, 1, 0, 0, K, 1, M, K);
@@ -101,7 +129,7 @@ static int linear_fwd_impl(const char* what, const float* ma, const float* Sa, c
   int rc = linear_fwd_check(what, ma, Sa, mw, Sw, Sz, M, K, N);
   if (rc != TAGI_OK) return rc;
   Plan p = linear_fwd_plan(M, K, N);
-  if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, M, N, 1))) p = choose_plan(M, N, K, 1, PROD_FWD, false, 1, nullptr, XD_A, linear_narrow(K, N));
+  if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, M, N, 1))) p = linear_fwd_plan(M, K, N, false);
   return linear_fwd_run(what, ma, Sa, mw, Sw, mb, Sb, mz, Sz, M, K, N, p, ws, ws_bytes, as_stream(stream), relu_J);
 }
 
@@ -147,7 +175,7 @@ static int linear_bwd_delta_impl(const char* what, const float* dmz, const float
   g.C = (int)K;
   g.Kred = (int)N;
   Plan p = linear_bwd_plan(M, K, N);
-  if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, M, K, 1))) p = choose_plan(M, K, N, 1, PROD_SHARED_B, false, 1, nullptr, XD_A, linear_narrow(K, N));
+  if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, M, K, 1))) p = linear_bwd_plan(M, K, N, false);
   const bool v4 = N % 4 == 0 && al16(dmz) && al16(dSz) && al16(mw);
   if (v4) return run_gemm<PROD_SHARED_B, LD_STR_K4, LD_STR_K4, 0, XD_A>(g, 1, p, ws, ws_bytes, s, what);
   return run_gemm<PROD_SHARED_B, LD_STR_K_S, LD_STR_K_S, 0, XD_A>(g, 1, p, ws, ws_bytes, s, what);
@@ -214,7 +242,7 @@ int linear_wgrad_impl(const char* what, const float* ma, const float* dmz, const
   g.Kred = (int)M;
   Plan p = linear_wgrad_plan(M, K, N);
   if (p.splits > 1 && (ws == nullptr || ws_bytes < plan_ws_bytes(p, K + 1, N, 1)))
-    p = choose_plan(K + 1, N, M, 1, PROD_SHARED_A, false, 1, nullptr, XD_B, linear_narrow(K, N));
+    p = linear_wgrad_plan(M, K, N, false);
   p.tiles_m = (int)cdiv(g.R, cfg_bm(p.cfg, p.xd));
   const bool v4 = K % 4 == 0 && N % 4 == 0 && al16(ma) && al16(dmz) && al16(dSz);
   if (mw) {

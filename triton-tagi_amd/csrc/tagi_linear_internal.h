@@ -7,7 +7,7 @@
 
 namespace tagi {
 
-Plan linear_fwd_plan(int64_t M, int64_t K, int64_t N);
+Plan linear_fwd_plan(int64_t M, int64_t K, int64_t N, bool split = true);
 Plan linear_fwd_plan32(int64_t M, int64_t K, int64_t N);
 
 int linear_fwd_check(const char* what, const float* ma, const float* Sa, const float* mw, const float* Sw,

@@ -42,6 +42,15 @@ class ConvGeom(ctypes.Structure):
     ]
 
 
+class Plan(ctypes.Structure):
+    """tagi_plan: the launch a Linear or Conv2D product gets."""
+
+    _fields_ = [
+        (n, c_int64)
+        for n in ("split_kernel", "tile_rows", "tile_cols", "tiles_rows", "tiles_cols", "splits", "k_chunk")
+    ]
+
+
 P = c_void_p
 I64 = c_int64
 F = c_float
@@ -56,6 +65,8 @@ class BnPending(ctypes.Structure):
 VP = POINTER(TagiView)
 GP = POINTER(ConvGeom)
 BP = POINTER(BnPending)
+PP = POINTER(Plan)
+OP_FWD, OP_FWD_FIXED, OP_BWD_DELTA, OP_WGRAD = range(4)  # TAGI_OP_*
 
 # name -> (restype, argtypes)
 _SIGS = {
@@ -68,6 +79,7 @@ _SIGS = {
     "tagi_probe_mfma_mix": (c_int, [P, I64, I64, c_int, c_int, P]),
     "tagi_probe_stream": (c_int, [P, P, I64, I64, c_int, P]),
     "tagi_probe_stream_variant": (c_int, [P, P, I64, I64, I64, c_int, c_int, c_int, P]),
+    "tagi_linear_plan": (c_int, [c_int, I64, I64, I64, I64, PP]),
     "tagi_linear_fwd": (c_int, [P, P, P, P, P, P, P, P, I64, I64, I64, P, I64, P]),
     "tagi_linear_fwd_relu": (c_int, [P, P, P, P, P, P, P, P, P, I64, I64, I64, P, I64, P]),
     "tagi_linear_fwd_ws_bytes": (I64, [I64, I64, I64]),
@@ -87,6 +99,7 @@ _SIGS = {
                                                 F, P]),
     "tagi_bmm_shared": (c_int, [P, P, P, P, P, I64, I64, I64, I64, VP, VP, VP, F, F, c_int, P]),
     "tagi_bmm_shared_jacobian": (c_int, [P, P, P, P, P, P, I64, I64, I64, I64, VP, VP, VP, F, F, c_int, P]),
+    "tagi_conv2d_plan": (c_int, [c_int, GP, I64, PP]),
     "tagi_conv2d_fwd": (c_int, [P, P, P, P, P, P, P, P, GP, P, I64, P]),
     "tagi_conv2d_fwd_ws_bytes": (I64, [GP]),
     "tagi_conv2d_fwd_relu_bn_stats": (c_int, [P, P, P, P, P, P, P, P, GP, P, P, P, P, P, P, F, F, c_int, c_int, P,
