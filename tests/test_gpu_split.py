@@ -12,8 +12,9 @@ EPS = 2.0**-24
 
 def bound(K, absum, squares):
     """Error of a K-term sum from the kernel: one rounding per 32-wide k tile (plus four for the
-    split-K partials and the epilogue) of sums no larger than the sum of magnitudes, one for each
-    product's omitted parts (below 2^-24 of it) and one for each squared operand."""
+    split-K partials and the epilogue) of sums no larger than the sum of magnitudes, one for the
+    omitted parts of the products (below 2^-24 of each), one for the truncation of the k tiles'
+    sums and one for each squared operand."""
     return (K / 32 + 6 + squares) * EPS * absum + 1e-37
 
 
@@ -137,3 +138,70 @@ def test_sums_over_many_rows_are_unbiased():
     # 2^24 outputs of independent roundings would leave 2^-12 of one rounding; the uncorrected
     # shift is 1e-8 of the outputs' size
     assert abs(err.mean().item()) < 1e-9 * d_ma.double().abs().mean().item()
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 8, 15, 16])
+def test_short_reductions(M):
+    """Parameter deltas of few rows: an error within fp32 arithmetic's own bound, one rounding
+    for each term and two for the variance's factor and its square."""
+    from triton_tagi_amd.layers import Linear
+
+    gen = torch.Generator("cuda").manual_seed(M)
+    torch.manual_seed(M)
+    K, N = 4096, 11008
+    layer = Linear(K, N, device="cuda")
+    for edge in (False, True):
+        ma, Sa = inputs((M, K), gen)
+        dm, dS = inputs((M, N), gen)
+        if edge:  # values whose split parts are the largest: just below 1 + 2^-7
+            ma, dm, dS = (1 + 2.0**-7 * (0.99 + 0.01 * torch.rand_like(t)) for t in (ma, dm, dS))
+        layer.forward(ma, Sa)
+        layer.backward(dm, dS)
+        a, V, d, e = (t.double() for t in (ma, layer.Sw, dm, dS))
+        for got, ref, mag, r in ((layer.delta_mw, V * (a.T @ d), V * (a.abs().T @ d.abs()), 1),
+                                 (layer.delta_Sw, V**2 * ((a**2).T @ e), V**2 * ((a**2).T @ e.abs()), 3)):
+            assert ((got.double() - ref).abs() / mag).max().item() < (M + r) * EPS
+
+
+@pytest.mark.parametrize("K", [24, 500, 1003])
+def test_constant_operands_leave_no_shift(K):
+    """Weights that are all alike (an initial variance), at the value whose split leaves out
+    the most: what is left out of the products averages out over the other operand."""
+    from triton_tagi_amd.layers import Linear
+
+    gen = torch.Generator("cuda").manual_seed(K)
+    M, N = 8192, 256
+    layer = Linear(K, N, bias=False, device="cuda")
+    layer.mw.fill_(1.0077972)
+    layer.Sw.fill_(1.0077972)
+    ma, Sa = inputs((M, K), gen)
+    for S in (Sa, None):
+        mz, Sz = layer.forward(ma, S)
+        w = layer.Sw.double()
+        ref = ma.double() ** 2 @ w + (0 if S is None else S.double() @ (w * w + w))
+        # columns alike: one number per row. A quarter of a rounding, three standard deviations
+        # of the mean of M rows' own roundings (K / 32 of them, up to one each), and the half
+        # that fp32 itself may round the constant mw^2 + Sw by
+        shift = ((Sz.double() - ref) / ref).mean().item()
+        own = 0.0 if S is None else 0.5
+        assert abs(shift) < EPS * (0.25 + own + 3 * (K / 32 + 2) ** 0.5 / M**0.5)
+
+
+@pytest.mark.parametrize("scale", [2.0**-90, 2.0**-105, 2.0**-112, 2.0**-120])
+def test_small_values(scale):
+    """Operands down to 2^-109 are split exactly; below, each is held to 2^-133."""
+    from triton_tagi_amd.layers import Linear
+
+    gen = torch.Generator("cuda").manual_seed(5)
+    torch.manual_seed(5)
+    M, K, N = 1000, 500, 516
+    layer = Linear(K, N, bias=False, device="cuda")
+    ma, Sa = inputs((M, K), gen, scale)
+    Sa *= scale
+    mz, Sz = layer.forward(ma, Sa)
+    a, S, w, V = (t.double() for t in (ma, Sa, layer.mw, layer.Sw))
+    fine = 2.0**-133  # per operand value, times the other operand
+    err = (mz.double() - a @ w).abs()
+    assert (err <= bound(K, a.abs() @ w.abs(), 0) + fine * w.abs().sum(0)).all()
+    err = (Sz.double() - (a**2 @ V + S @ (w**2 + V))).abs()
+    assert (err <= bound(2 * K, a**2 @ V + S @ (w**2 + V), 2) + fine * (2 * V + w**2).sum(0) + 2.0**-126).all()

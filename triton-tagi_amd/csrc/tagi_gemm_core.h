@@ -2148,9 +2148,12 @@ struct Plan {
 //     3 input at 131072 pixels 28.9 against 33.3 us), and input deltas of more than 64
 //     channels (137 <- 362 channels, stride 2, with its other products 256 against 290; 42 <-
 //     70 channels 44.5 against 40.5);
-//   * sides under 4, which its float4 loads of any alignment do not cover.
+//   * sides under 4, which its float4 loads of any alignment do not cover;
+//   * reductions under 16: a k tile's partial sums are truncated and not rounded, which is
+//     made up for only where many terms share the tile (one term: 0.8 units of 2^-24 rms and
+//     5.6 at most against 0.6 and 2; four terms: 0.46 against 0.53 rms, eight 0.3 against 0.4).
 static inline bool use_split(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, int xd, bool narrow) {
-  if (xd == XD_NONE || narrow) return false;
+  if (xd == XD_NONE || narrow || Kred < 16) return false;
   const double macs = (double)R * C * Kred * batch;
   if (macs < (double)(1 << 25) || (Kred >= 256 && macs < (double)(1 << 26))) return false;
   return !(xd & XD_SCALAR) || (prod == PROD_SHARED_B ? C <= 64 : Kred >= 32);
