@@ -64,7 +64,7 @@ static int check_geom(const tagi_conv_geom* g, const char* what) {
 static Plan conv_fwd_plan(const tagi_conv_geom* g, bool zero_var = false, bool split = true) {
   // (the split kernel's patch loads take up to 25 taps)
   return choose_plan(g->N * g->Ho * g->Wo, g->Cout, g->C * g->k * g->k, 1, zero_var ? PROD_SHARED_A : PROD_FWD, split,
-                     split ? 16 : 1, nullptr, XD_A | (g->C % 4 ? XD_SCALAR : 0), g->Cout < 4 || g->k > 5);
+                     split ? 16 : 1, nullptr, XD_A | XD_PATCH | (g->C % 4 || g->Cout % 4 ? XD_SCALAR : 0), g->Cout < 4 || g->k > 5);
 }
 
 // Largest row count (phase 0) and largest reduction over the stride phases of the
@@ -89,7 +89,7 @@ static Plan conv_bwd_plan(const tagi_conv_geom* g, bool split = true) {
   const ConvG cg = to_g(g);
   const int nph = cg.stride * cg.stride;
   int64_t pk[64];
-  const int xd = XD_A | (g->Cout % 4 ? XD_SCALAR : 0);
+  const int xd = XD_A | XD_PATCH | (g->Cout % 4 ? XD_SCALAR : 0);
   const bool narrow = g->C < 4 || g->k > 5;
   if (!split || nph > 64)
     return choose_plan(R, g->C, K, nph, PROD_SHARED_B, split, split ? 16 : 1, nullptr, xd, narrow);
@@ -103,7 +103,7 @@ static Plan conv_bwd_plan(const tagi_conv_geom* g, bool split = true) {
 // rows: the weight rows (c, kh, kw), plus the ones row of the bias sums when the GEMM forms them
 static Plan conv_wgrad_plan(const tagi_conv_geom* g, bool bias, bool split = true) {
   return choose_plan(g->C * g->k * g->k + (bias ? 1 : 0), g->Cout, g->N * g->Ho * g->Wo, 1, PROD_SHARED_A, split,
-                     split ? 512 : 1, nullptr, XD_B, g->Cout < 4);
+                     split ? 512 : 1, nullptr, XD_B | XD_PATCH, g->Cout < 4);
 }
 
 extern "C" int tagi_conv2d_plan(int op, const tagi_conv_geom* g, int64_t ws_bytes, tagi_plan* out) {

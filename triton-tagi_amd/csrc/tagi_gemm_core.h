@@ -2122,8 +2122,9 @@ static const CfgDesc kCfg[] = {{128, 128, 16}, {128, 64, 16}, {64, 128, 16}, {64
                                {64, 64, 32},   {128, 32, 32},  {64, 32, 32},  {32, 32, 32}};
 static const int kNumCfg32 = 6, kNumCfg = 14;
 // which operand the split kernel reads directly (0: the product has no split kernel)
-// (XD_SCALAR, with XD_A: that operand's conv patches are read element by element)
-enum { XD_NONE = 0, XD_A = 1, XD_B = 2, XD_SCALAR = 4 };
+// (XD_PATCH: a conv's product; XD_SCALAR, with XD_A: its patches are read element by element;
+// XD_ANY: Linear rows that float4 loads do not divide)
+enum { XD_NONE = 0, XD_A = 1, XD_B = 2, XD_SCALAR = 4, XD_ANY = 8, XD_PATCH = 16 };
 static inline int cfg_bm(int c, int xd) { return c >= kNumCfg32 && xd == XD_B ? kCfg[c].BN : kCfg[c].BM; }
 static inline int cfg_bn(int c, int xd) { return c >= kNumCfg32 && xd == XD_B ? kCfg[c].BM : kCfg[c].BN; }
 
@@ -2135,9 +2136,18 @@ struct Plan {
   int xd;  // the call's direct operand (XD_*)
 };
 
-// Whether a product with a split kernel runs it (else the fp32 kernel). The split kernel is
-// the faster one wherever the matrix cores or the loads' volume bound the launch, 1.2 to 1.8
-// times at 2^28 multiply-adds and more. Not on
+// Whether a product with a split kernel runs it (else the fp32 kernel). The fp32 kernel's time
+// over the split kernel's, each in its planner's choice, over 3500 random Linear and Conv2D
+// shapes of 2^25 to 2^33 multiply-adds: 1.11 (geometric mean), by product and reduction
+//   Linear, 128 and longer    forward 1.18, fixed input 1.24, input deltas 1.11, parameters 1.12
+//   Linear, 48 to 127         forward 1.11, fixed input 1.09, input deltas 1.08, parameters 1.03
+//   Linear, under 48          forward 1.04, fixed input 0.96, input deltas 0.95, parameters 0.89
+//   Conv2D, float4 patches    forward 1.09, fixed input 1.12, input deltas 1.13, parameters 1.06
+//   Conv2D, element-wise      forward 1.01, fixed input 1.13, input deltas 1.10, parameters 1.20
+// The products that lose stay, as the closer ones to float64 (2 to 4 times from reductions of 64
+// on): element-wise patches beside 32 columns and fewer (forward 0.54 to 0.86, input deltas over
+// 1024 and more 0.57 to 0.98), aligned parameter deltas of 16 and 32 columns at 2^29 and more
+// (0.67 to 1.0), few rows' parameter deltas of very wide layers (0.7 to 0.9). Not on
 //   * products whose launch, loads' latency and barriers are the time: under 2^25
 //     multiply-adds (the kernels tie within 2 us when repeated, but the split kernel's longer
 //     code is fetched anew in a step of many kernels: MLP steps of batch 42 and 72 2-4%
@@ -2146,17 +2156,43 @@ struct Plan {
 //     its parameter deltas 13.8 against 14.7);
 //   * element-wise patches, whose decode is the time in both: under one k tile (a 3-channel 3 x
 //     3 input at 131072 pixels 28.9 against 33.3 us), and input deltas of more than 64
-//     channels (137 <- 362 channels, stride 2, with its other products 256 against 290; 42 <-
-//     70 channels 44.5 against 40.5);
+//     channels (0.9 to 1.15 over 66 to 408 channels, 0.6 to 0.8 where 128 x 128 tiles run);
 //   * sides under 4, which its float4 loads of any alignment do not cover;
-//   * reductions under 16: a k tile's partial sums are truncated and not rounded, which is
-//     made up for only where many terms share the tile (one term: 0.8 units of 2^-24 rms and
-//     5.6 at most against 0.6 and 2; four terms: 0.46 against 0.53 rms, eight 0.3 against 0.4).
+//   * reductions under 4: a k tile's partial sums are truncated and not rounded, which is
+//     made up for only where terms share the tile (rms and largest error in units of 2^-24,
+//     fp32 kernel first: one term 0.60 and 2.0 against 0.72 and 3.4, two 0.56 and 2.8 against
+//     0.59 and 3.5, four 0.45 and 3.2 against 0.36 and 2.6).
 static inline bool use_split(int64_t R, int64_t C, int64_t Kred, int64_t batch, int prod, int xd, bool narrow) {
-  if (xd == XD_NONE || narrow || Kred < 16) return false;
+  if (xd == XD_NONE || narrow || Kred < 4) return false;
   const double macs = (double)R * C * Kred * batch;
   if (macs < (double)(1 << 25) || (Kred >= 256 && macs < (double)(1 << 26))) return false;
   return !(xd & XD_SCALAR) || (prod == PROD_SHARED_B ? C <= 64 : Kred >= 32);
+}
+
+// Split tiles left out (bit x: tile kNumCfg32 + x): the time model below does not know of
+// registers spilled by a loader, nor what the exposed prologue and epilogue of a block alone on
+// its CU cost a short reduction. In brackets the fp32 kernel's time over such a tile's, and
+// over the time of the tile chosen instead (every tile forced in turn on 180 such products,
+// and 3500 random Linear and Conv2D shapes before and after).
+static inline unsigned split_skip(int64_t Kred, int prod, int xd) {
+  enum { T256x128 = 1, T256x64 = 2, T128x128 = 4, T128x64 = 8, T128x32 = 32 };
+  const bool wgrad = xd & XD_B;
+  unsigned m = 0;
+  // Linear rows of any alignment: forward 256 x 128 0.71 (1.22), fixed inputs 256 x 128 and 128
+  // x 128 0.92 (1.28), input deltas 128 x 128 0.83 (1.17), parameter deltas 128 x 128 0.56 (1.12)
+  if (xd & XD_ANY)
+    m |= prod == PROD_FWD ? T256x128 : prod == PROD_SHARED_B || wgrad ? T128x128 : T256x128 | T128x128;
+  // element-wise patches: forward 128 x 64 and 128 x 32 0.62 to 0.82 (0.72 to 1.0), fixed inputs
+  // 128 x 128 0.90 (1.2), input deltas 128 x 32, 128 x 128 and 256 x 128 0.22 to 0.75 (0.6 to 1.1)
+  if (xd & XD_SCALAR)
+    m |= prod == PROD_FWD ? T128x64 | T128x32 : prod == PROD_SHARED_B ? T256x128 | T128x128 | T128x32 : T128x128;
+  // short reductions: forward 0.8 to 1.0 (1.0 to 1.15 in 64 x 64), fixed inputs 0.8 to 0.97 (1.0
+  // to 1.1), input deltas 0.78 to 0.98 in 256 rows (1.1 to 1.3 in 128 x 128), parameter deltas
+  // 0.5 to 0.95 (0.8 to 1.1)
+  if (Kred < (wgrad ? 256 : 128)) m |= T256x128 | T256x64;
+  if (prod == PROD_SHARED_B || (xd & XD_PATCH)) return m;
+  if (Kred < (wgrad ? 256 : prod == PROD_FWD ? 128 : 64)) m |= T128x128 | T128x64;
+  return m;
 }
 
 // The split kernel's plan, from the same kind of model as the fp32 kernel's below: blocks run
@@ -2193,9 +2229,11 @@ static inline Plan choose_split_plan(int64_t R, int64_t C, int64_t Kred, int64_t
   const double kFixed = 0.24e-6, kOut = 4.26e-10, kDecode = 3.52e-10, kSplitSecPerByte = 1.25e-13, kSplitLaunch = 2.0e-6;
   const int products = prod == PROD_FWD ? 3 : 2;
   const int side = xd & (XD_A | XD_B);
+  const unsigned skip = split_skip(Kred, prod, xd);
   Plan best{};
   double best_t = DBL_MAX;
   for (int x = 0; x < kNumCfg - kNumCfg32; ++x) {
+    if ((skip >> x) & 1u) continue;
     const int ci = kNumCfg32 + x, BM = cfg_bm(ci, side), BN = cfg_bn(ci, side), bpc = kBpc[x][prod];
     const int64_t tm = cdiv(R, BM), tn = cdiv(C, BN);
     int64_t prev = -1;
@@ -2346,7 +2384,7 @@ static inline Plan choose_plan(int64_t R, int64_t C, int64_t Kred, int64_t batch
   };
   static thread_local Entry cache[64];
   static thread_local int used = 0, next = 0;
-  const Key key{R, C, Kred, batch, max_splits, salt, prod, allow_split ? 1 : 0, xd + (narrow ? 8 : 0)};
+  const Key key{R, C, Kred, batch, max_splits, salt, prod, allow_split ? 1 : 0, xd + (narrow ? 32 : 0)};
   for (int i = 0; i < used; ++i) {
     const Key& k = cache[i].k;
     if (k.R == R && k.C == C && k.K == Kred && k.batch == batch && k.max_splits == max_splits && k.salt == salt &&

@@ -7,6 +7,8 @@ static inline hipStream_t as_stream(tagi_stream_t s) { return (hipStream_t)s; }
 
 // layer widths under one float4 (kept off the split kernel)
 static bool linear_narrow(int64_t K, int64_t N) { return K < 4 || N < 4; }
+// the direct operand and whether float4 loads divide the rows
+static int linear_xd(int side, int64_t K, int64_t N) { return side | (K % 4 || N % 4 ? XD_ANY : 0); }
 
 // The forward's plan over a reduction of the fp32 kernel alone: what tagi_linear_fwd_noalloc
 // accepts is decided by its workspace.
@@ -14,26 +16,26 @@ Plan tagi::linear_fwd_plan32(int64_t M, int64_t K, int64_t N) { return choose_pl
 
 // split: whether the reduction may be cut (the caller's workspace holds the partial sums)
 Plan tagi::linear_fwd_plan(int64_t M, int64_t K, int64_t N, bool split) {
-  const Plan p = choose_plan(M, N, K, 1, PROD_FWD, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
+  const Plan p = choose_plan(M, N, K, 1, PROD_FWD, split, split ? 16 : 1, nullptr, linear_xd(XD_A, K, N), linear_narrow(K, N));
   constexpr int64_t kScratch = TAGI_LINEAR_FWD_NOALLOC_SCRATCH_BYTES;
   if (plan_ws_bytes(p, M, N, 1) <= kScratch || plan_ws_bytes(linear_fwd_plan32(M, K, N), M, N, 1) > kScratch) return p;
   // the fixed scratch holds every shape that tagi_linear_fwd_noalloc accepts: fewer splits,
   // none where one pair of partial planes is already larger (M N > 2^24)
   const int64_t fit = kScratch / (8 * M * N);
-  return choose_plan(M, N, K, 1, PROD_FWD, fit > 1, fit > 1 ? fit : 1, nullptr, XD_A, linear_narrow(K, N));
+  return choose_plan(M, N, K, 1, PROD_FWD, fit > 1, fit > 1 ? fit : 1, nullptr, linear_xd(XD_A, K, N), linear_narrow(K, N));
 }
 static Plan linear_bwd_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
-  return choose_plan(M, K, N, 1, PROD_SHARED_B, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
+  return choose_plan(M, K, N, 1, PROD_SHARED_B, split, split ? 16 : 1, nullptr, linear_xd(XD_A, 0, N), linear_narrow(K, N));
 }
 static Plan linear_wgrad_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
-  return choose_plan(K + 1, N, M, 1, PROD_SHARED_A, split, split ? 512 : 1, nullptr, XD_B, linear_narrow(K, N));
+  return choose_plan(K + 1, N, M, 1, PROD_SHARED_A, split, split ? 512 : 1, nullptr, linear_xd(XD_B, K, N), linear_narrow(K, N));
 }
 
 // A deterministic input (no variance, Sa NULL): mean = ma mw, variance = ma^2 Sw, the
 // shared-A product (two MFMAs per k-step instead of three; the terms Sa (mw^2 + Sw) it
 // leaves out are exact zeros)
 static Plan linear_fwd0_plan(int64_t M, int64_t K, int64_t N, bool split = true) {
-  return choose_plan(M, N, K, 1, PROD_SHARED_A, split, split ? 16 : 1, nullptr, XD_A, linear_narrow(K, N));
+  return choose_plan(M, N, K, 1, PROD_SHARED_A, split, split ? 16 : 1, nullptr, linear_xd(XD_A, K, N), linear_narrow(K, N));
 }
 
 extern "C" int tagi_linear_plan(int op, int64_t M, int64_t K, int64_t N, int64_t ws_bytes, tagi_plan* out) {
