@@ -218,12 +218,22 @@ def test_conv_bwd_delta_with_addend(dev, case):
 
 
 FOLD_CASES = [
-    # N, C_in (the BatchNorm2D channels), H, W, C_out, k: shapes whose input-delta plan
-    # is unsplit with one tile per wave (the fold's condition)
+    # N, C_in (the BatchNorm2D channels), H, W, C_out, k: shapes whose input-delta plan is
+    # unsplit, in a tile that carries the fold (one 32 x 32 tile per wave of the fp32 kernel, any
+    # tile of the split kernel)
     (16, 64, 32, 32, 64, 3),  # ResNet-18 stage 1 at batch 16
     (16, 6, 16, 16, 8, 3),    # C_in off the float4 path
     (8, 12, 12, 10, 16, 3),   # C_out below the tile-aligned loaders' 16
     (8, 32, 8, 8, 16, 1),
+    # the split kernel, each tile with whole k tiles per tap (C_out a multiple of 32) and without
+    (11, 240, 9, 9, 160, 1), (6, 283, 9, 9, 28, 3),      # 32 x 32
+    (83, 76, 10, 10, 64, 1), (33, 6, 31, 31, 8, 5),      # 64 x 32
+    (19, 168, 15, 15, 64, 1), (94, 35, 17, 17, 4, 3),    # 64 x 64
+    (46, 286, 12, 12, 32, 1), (141, 5, 24, 24, 4, 5),    # 128 x 32
+    (7, 228, 30, 30, 32, 1), (84, 227, 10, 10, 24, 1),   # 128 x 64
+    (74, 196, 14, 14, 32, 1), (40, 245, 19, 19, 28, 1),  # 128 x 128
+    (127, 50, 20, 20, 32, 3), (48, 33, 34, 34, 8, 5),    # 256 x 64
+    (39, 224, 26, 26, 128, 1), (116, 75, 23, 23, 16, 3), # 256 x 128
 ]
 
 
