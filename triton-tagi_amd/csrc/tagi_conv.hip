@@ -387,7 +387,7 @@ static int conv_bwd_delta_impl(const char* what, const float* dmz, const float* 
   if (p.splits > 1 && part_bytes < plan_ws_bytes(p, R0, g->C, nph)) p = conv_bwd_plan(g, false);
   if (bnf) {
     TAGI_REQUIRE(nph == 1 && p.splits == 1 && bnf_cfg(p.cfg),
-                 "%s: the folded BatchNorm2D backward needs stride 1 and an unsplit one-tile-per-wave plan", what);
+                 "%s: the folded BatchNorm2D backward needs stride 1 and an unsplit plan in a tile that carries it", what);
     // the folded epilogues address the (N, H, W, C) tensors with 32-bit offsets
     TAGI_REQUIRE(R0 * g->C < (int64_t)1 << 31, "%s: %lld x %lld deltas exceed the fold's 2^31 elements", what,
                  (long long)R0, (long long)g->C);

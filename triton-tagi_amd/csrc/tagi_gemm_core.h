@@ -2437,10 +2437,11 @@ static inline tagi_plan plan_info(const Plan& p) {
   X(PROD_SHARED_A, LD_STR_MN4, LD_STR_K4)
 
 // The input-delta loader pairs that also get the folded BatchNorm2D epilogues (EPI 1 and
-// 3), in the tile configs with one 32 x 32 tile per wave (64 x 64, 32 x 32, 128 x 32)
+// 3): in the fp32 kernel's tile configs with one 32 x 32 tile per wave (64 x 64, 32 x 32,
+// 128 x 32), and in every split tile
 #define TAGI_GEMM_COMBOS_SHARED_B_BNF(X)                                                 \
   X(PROD_SHARED_B, LD_CBWD_A4T, LD_CBWD_BK4T) X(PROD_SHARED_B, LD_CBWD_A4, LD_CBWD_BK4)
-static inline bool bnf_cfg(int cfg) { return cfg >= 3; }
+static inline bool bnf_cfg(int cfg) { return cfg >= kNumCfg32 || cfg == 3 || cfg == 4 || cfg == 5; }
 // The Linear parameter-delta loader pairs that also get the in-place update (EPI 2), in
 // every tile config
 #define TAGI_GEMM_COMBOS_SHARED_A_UPD(X)                                                 \
@@ -2511,7 +2512,7 @@ template <int PROD, int KA, int KB, int EPI = 0, int XD = XD_NONE>
 static inline int run_gemm(GemmArgs g, int64_t batch, const Plan& p, float* ws, int64_t ws_bytes, hipStream_t s,
                            const char* what, int64_t grid_x_override = 0) {
   if constexpr (EPI == 1 || EPI == 3)
-    TAGI_REQUIRE(bnf_cfg(p.cfg) && p.splits == 1, "%s: folded epilogue needs an unsplit one-tile-per-wave plan",
+    TAGI_REQUIRE(bnf_cfg(p.cfg) && p.splits == 1, "%s: folded epilogue needs an unsplit plan in a tile that carries it",
                  what);
   // operand byte offsets are 32-bit with the out-of-range sentinel above them
   TAGI_REQUIRE(g.a.nbytes >= 0 && g.a.nbytes < (int64_t)kBufOutOfRange && g.b.nbytes >= 0 &&
@@ -2538,6 +2539,9 @@ static inline int run_gemm(GemmArgs g, int64_t batch, const Plan& p, float* ws, 
   if (p.cfg >= kNumCfg32) {
     if constexpr (XD != XD_NONE) {
       TAGI_REQUIRE(p.xd == XD && (p.splits == 1 || p.k_chunk % 32 == 0), "%s: internal: plan of another call", what);
+      // each split kernel holds one kind of epilogue, the plain store without a bias per row
+      constexpr int kind = XD == XD_B ? 1 : (KA == LD_CBWD_A4 || KA == LD_CBWD_A_S || KA == LD_CBWD_A4T) ? 2 : 0;
+      TAGI_REQUIRE(g.epi.kind == kind && g.epi.b_sr == 0, "%s: internal: no split kernel with this epilogue", what);
       // EPI 2 and 4 apply their epilogue in the kernel only when unsplit, as below
       constexpr int E0 = (EPI == 2 || EPI == 4) ? 0 : EPI;
       constexpr int NA = any_kind(KA), NB = any_kind(KB), UA = untiled_kind(KA), UB = untiled_kind(KB);
