@@ -32,13 +32,19 @@ sys.path.insert(0, str(ROOT))
 
 METRIC = "TAGI step samples/sec (fwd+bwd+update) ResNet-18 b128 fp32; % MFMA/HBM peak"
 PEAK_FP32_MFMA_TFLOPS = 157.3
-# Linear and Conv2D products run as six bf16 part products each (dense bf16 peak / 6)
+# Linear and Conv2D products run as six bf16 part products each (dense bf16 peak / 6), but for
+# the small ones, which run the fp32 MFMA
 PEAK_SPLIT_TFLOPS = 419.4
+SPLIT_MIN_MACS = 1 << 25
 PEAK_HBM_GBS = 8000.0
 
 
-def mfma_peak(family: str) -> float:
-    return PEAK_SPLIT_TFLOPS if family.startswith(("conv_", "linear_")) else PEAK_FP32_MFMA_TFLOPS
+def mfma_peak(family: str, flops_per_launch: float) -> float:
+    """Peak of the kernel that a family's launches run, by their mean size (multiply-adds of one
+    of the two or, in a forward, three products)."""
+    macs = flops_per_launch / (6 if family.endswith("_fwd") else 4)
+    split = family.startswith(("conv_", "linear_")) and macs >= SPLIT_MIN_MACS
+    return PEAK_SPLIT_TFLOPS if split else PEAK_FP32_MFMA_TFLOPS
 
 
 TIMER_STEPS = 5  # timed steps (the last ones) that carry the live per-launch timer
@@ -495,11 +501,12 @@ def main():
         # (fp32 MFMA 157.3 TFLOP/s / 8 TB/s = 19.7 flop/B, bf16 parts 52.4): products with a short reduction (the
         # attention score products, K = head_dim) are bound by moving their outputs
         hbm_bound = bytes_per_launch > 0 and flops_per_launch / bytes_per_launch < (
-            mfma_peak(dom) * 1e12 / (PEAK_HBM_GBS * 1e9))
+            mfma_peak(dom, flops_per_launch) * 1e12 / (PEAK_HBM_GBS * 1e9))
         if hbm_bound:
             achieved, peak, unit = bytes_per_launch / per_launch_s / 1e9, PEAK_HBM_GBS, "GB/s"
         else:
-            achieved, peak, unit = flops_per_launch / per_launch_s / 1e12, mfma_peak(dom), "TFLOP/s"
+            achieved, unit = flops_per_launch / per_launch_s / 1e12, "TFLOP/s"
+            peak = mfma_peak(dom, flops_per_launch)
         roofline = {
             "bound": "hbm" if hbm_bound else "mfma",
             "kernel": dom,
@@ -522,7 +529,7 @@ def main():
         e = {"ms_per_step": round(v["ms"] / nps, 4), "launches_per_step": v["launches"] / nps}
         if v["flops"]:
             e["tflops"] = round(v["flops"] / (v["ms"] / 1e3) / 1e12, 2)
-            e["mfma_frac"] = round(e["tflops"] / mfma_peak(f), 4)
+            e["mfma_frac"] = round(e["tflops"] / mfma_peak(f, v["flops"] / v["launches"]), 4)
         elif v["bytes"]:
             e["gbs"] = round(v["bytes"] / (v["ms"] / 1e3) / 1e9, 1)
             e["hbm_frac"] = round(e["gbs"] / PEAK_HBM_GBS, 4)
