@@ -19,10 +19,10 @@
 // memory to registers in the MFMA's fragment layout, each wave owning its rows of it; the
 // other (staged) is split by the whole block and shared through LDS as bf16 parts. 16x16x32
 // MFMAs, which sustain 2.1 PF/s here where 32x32x16 throttles at 1.85 (random operands).
-// Measured with the fp32 kernel's best tile on the left (4096 x 4096 x 4096): forward 2984 ->
-// 1929 us (214 TF/s of fp32 products), input deltas 1964 -> 1231, parameter deltas 2225 ->
-// 1540; a 64-channel 3 x 3 Conv2D at 131072 pixels: forward 254 -> 191, input deltas 184 ->
-// 140, parameter deltas 184 -> 155 (one run; the layer 584 -> 487).
+// Measured, fp32 kernel on the left, each in its plan (4096 x 4096 x 4096, one run): forward
+// 3021 -> 2166 us (190 TF/s of fp32 products), input deltas 2036 -> 1389, parameter deltas 2107
+// -> 1750; a 64-channel 3 x 3 Conv2D at 131072 pixels: forward 246 -> 193, input deltas 183 ->
+// 152, parameter deltas 197 -> 170.
 #pragma once
 #include "tagi_gemm_core.h"
 
@@ -108,8 +108,9 @@ __global__ void __launch_bounds__(X::NTH, (split_minw<PROD, X, KA, KB>())) gemm_
   using LD = Loader<DA ? KA : KB, ND, NW * DM, BK, NTH, 1, 2, DM>;
   using LS = Loader<DA ? KB : KA, NL, LM, BK, NTH, 1, 1>;
   // LDS: [buffer][product][part][k / 8][row][8 bf16]; the k / 8 planes are offset by 64
-  // bytes and the rows of a group of four permuted (phys below) so that the stores of every
-  // unit shape and the fragment reads touch each bank once
+  // bytes and the rows of a group of four permuted (phys below), which spreads the stores of
+  // every unit shape over the banks (the counters still read half of the LDS cycles as
+  // conflicts, at one LDS instruction per 8 to 18 VALU instructions)
   constexpr int QS = LM * 16 + 64, PS = 4 * QS, BUF = NP * 3 * PS;
   constexpr int RAW = NL * LM * BK * 4;  // fp32 tile of the fallback loop
   constexpr int SM = NBUF * BUF > RAW ? NBUF * BUF : RAW;

@@ -2,7 +2,7 @@
 
 Drop-in for the step path of triton-tagi: the same layer classes, ``Sequential.step``
 and update rules, with every moment computation in hand-written HIP kernels for gfx950
-(fp32 MFMA for the moment GEMMs) behind the C ABI of ``libtagi_hip.so``.
+(matrix cores for the moment GEMMs, fp32 operands and results) behind the C ABI of ``libtagi_hip.so``.
 """
 
 from .base import Layer, LearnableLayer

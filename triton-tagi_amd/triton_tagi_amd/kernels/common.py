@@ -4,8 +4,9 @@
     backward: dma = dmz @ mw^T,   dSa = dSz @ (mw^2)^T
     deltas:   gmw = ma^T @ dmz,   gSw = (ma^2)^T @ dSz
 
-Each is one fp32-MFMA kernel launch (two accumulators) behind the C ABI; the
-``triton_*`` names of the reference are kept as aliases.
+Each is one moment-GEMM launch (two accumulators, fp32 operands and results, plus a reduction
+where its sums are cut up) behind the C ABI; the ``triton_*`` names of the reference are kept as
+aliases.
 """
 
 from __future__ import annotations

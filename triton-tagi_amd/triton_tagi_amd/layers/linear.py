@@ -1,6 +1,6 @@
 """Bayesian Linear layer (mirrors triton_tagi/layers/linear.py:30-181).
 
-Forward (one fused fp32-MFMA launch):
+Forward (one fused moment-GEMM launch):
     mu_z = mu_a @ mu_w + mu_b
     S_z  = mu_a^2 @ S_w + S_a @ (mu_w^2 + S_w) + S_b
 Backward (deltas stored, applied by ``update``, or by the backward pass itself within
