@@ -252,7 +252,7 @@ def same_specials(got, ref, what):
 
 
 # (64, 64, 64) runs the fp32 kernel, the others the split kernel in every product
-@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (3000, 100, 1130), (730, 700, 1001)])
+@pytest.mark.parametrize("M,K,N", [(64, 64, 64), (3000, 100, 1130), (130, 700, 1001), (730, 700, 1001)])
 def test_infinities_and_nan(M, K, N):
     """Infinite, NaN and huge operands: the outputs they reach are those of fp32 arithmetic, the
     others are unharmed (their tile is formed again by fp32 MFMAs, so their rounding may change)."""

@@ -93,10 +93,12 @@ def test_products_that_stay_with_the_fp32_kernel():
     conv = [
         (F, (128, 3, 32, 64, 3, 1), (128, 5, 32, 64, 3, 1)),  # element-wise patches under one k tile
         (D, (50, 66, 27, 70, 3, 1), (50, 62, 27, 70, 3, 1)),  # and their input deltas of many channels
+        (D, (200, 64, 64, 3, 3, 2), (200, 64, 64, 4, 3, 2)),  # a stride phase of too few terms
     ]
     for op, a, b in conv:
-        assert conv_plan(op, geom(*a)).split_kernel == 0, (op, a)
-        assert conv_plan(op, geom(*b)).split_kernel == 1, (op, b)
+        for ws in (-1, 0):
+            assert conv_plan(op, geom(*a), ws).split_kernel == 0, (op, a)
+            assert conv_plan(op, geom(*b), ws).split_kernel == 1, (op, b)
 
 
 def test_tiles_left_out():

@@ -90,13 +90,14 @@ static Plan conv_bwd_plan(const tagi_conv_geom* g, bool split = true) {
   const int nph = cg.stride * cg.stride;
   int64_t pk[64];
   const int xd = XD_A | XD_PATCH | (g->Cout % 4 ? XD_SCALAR : 0);
-  const bool narrow = g->C < 4 || g->k > 5;
-  if (!split || nph > 64)
-    return choose_plan(R, g->C, K, nph, PROD_SHARED_B, split, split ? 16 : 1, nullptr, xd, narrow);
-  for (int ph = 0; ph < nph; ++ph) {
+  bool narrow = g->C < 4 || g->k > 5;
+  for (int ph = 0; ph < nph && ph < 64; ++ph) {
     const Phase p = make_phase(cg, ph);
     pk[ph] = (int64_t)p.nkh * p.nkw * g->Cout;
+    narrow |= pk[ph] > 0 && pk[ph] < 4;  // (the shortest reduction of the split kernel)
   }
+  if (!split || nph > 64)
+    return choose_plan(R, g->C, K, nph, PROD_SHARED_B, split, split ? 16 : 1, nullptr, xd, narrow);
   return choose_plan(R, g->C, K, nph, PROD_SHARED_B, true, 16, pk, xd, narrow);
 }
 
